@@ -10,6 +10,7 @@
 // (saveMagneticFields) and B_m <- (B + B_m)/2 (centerMagneticFields) are
 // fused into the Faraday kernel.
 #include "kernels.h"
+#include "pic_device.h"
 
 namespace smi {
 
@@ -197,35 +198,76 @@ __global__ void k_ukin(PartPtrs A, const int32_t *__restrict__ perm, int64_t n, 
 }
 
 // Charge density, shape of the interpolation order (Projector3D2Order::
-// basic type 0, Projector3D2Order.cpp:526-621), FP64 atomics, periodic.
+// basic type 0, Projector3D2Order.cpp:526-621), FP64, periodic.  One
+// workgroup per 4^ND cluster of the sorted list: the nearest node of its
+// particles is one of 5 per axis, so their stencils span a tile of 5 + 2H
+// points per axis, summed with LDS atomics and flushed once.  Adding every
+// contribution to global memory instead was bound by the memory-side FP64
+// atomics (27 or 125 per particle, 3e10/s): mean 1.71 ms over species of
+// 2.4e6, 2.4e6 and 6.2e5 particles at order 2, 1.70 ms for 4.1e5 at order 4,
+// 1.30 ms for 4.2e6 in 2D, against 0.053, 0.059 and 0.036 ms for the tile.  A node outside the tile (a position its key does
+// not describe) goes to global memory directly.
 template <int ND, int ORDER>
-__global__ void k_rho(Geom g, SpeciesK sp, PartPtrs A, const int32_t *__restrict__ perm, int64_t n,
-                      double *__restrict__ rho)
+__global__ void __launch_bounds__(256)
+k_rho(Geom g, SpeciesK sp, PartPtrs A, const int32_t *__restrict__ perm, const int32_t *__restrict__ cell_off,
+      double *__restrict__ rho)
 {
-    constexpr int H = ORDER / 2, W = 2 * H + 1;
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const int i = perm[j];
-    const double x[3] = {A.x[i], A.y[i], ND == 3 ? A.z[i] : 0.};
-    double S[3][5];
-    int o[3] = {0, 0, 0};
-    for (int d = 0; d < ND; ++d) {
-        const double pn = x[d] * g.dinv[d];
-        if (!(pn > -4.0 && pn < g.N[d] + 4.0)) return;  // outside the box: not deposited
-        const int ip = (int)round(pn);
-        spline<ORDER>(pn - (double)ip, S[d]);
-        o[d] = ip - H;
-    }
-    const double cw = sp.cw_scale * A.w[i];
-    for (int a = 0; a < W; ++a)
-        for (int b = 0; b < W; ++b) {
-            if constexpr (ND == 3) {
-                for (int c = 0; c < W; ++c)
-                    unsafeAtomicAdd(&rho[lin(g, o[0] + a, o[1] + b, o[2] + c)], cw * S[0][a] * S[1][b] * S[2][c]);
-            } else {
-                unsafeAtomicAdd(&rho[lin(g, o[0] + a, o[1] + b, 0)], cw * S[0][a] * S[1][b]);
-            }
+    constexpr int H = ORDER / 2, W = 2 * H + 1, T = 5 + 2 * H, TN = ND == 3 ? T * T * T : T * T;
+    __shared__ double sR[TN];
+    const dev::Cluster cl = dev::decode_cluster(g, blockIdx.x);
+    const int s = cell_off[cl.gbase], e = cell_off[cl.gbase + g.cells_per_cl];
+    if (s == e) return;  // uniform across the workgroup
+    for (int t = threadIdx.x; t < TN; t += blockDim.x) sR[t] = 0.;
+    __syncthreads();
+    for (int j = s + (int)threadIdx.x; j < e; j += blockDim.x) {
+        const int i = perm[j];
+        const double x[3] = {A.x[i], A.y[i], ND == 3 ? A.z[i] : 0.};
+        double S[3][5];
+        int o[3] = {0, 0, 0};
+        bool box = true, tile = true;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            const double pn = x[d] * g.dinv[d];
+            box &= pn > -4.0 && pn < g.N[d] + 4.0;
+            const int ip = (int)round(pn);
+            spline<ORDER>(pn - (double)ip, S[d]);
+            o[d] = ip - cl.G0[d];
+            tile &= o[d] >= 0 && o[d] <= 4;
         }
+        if (!box) continue;  // outside the box: not deposited
+        const double cw = sp.cw_scale * A.w[i];
+        if (!tile) {
+            for (int a = 0; a < W; ++a)
+                for (int b = 0; b < W; ++b)
+                    for (int c = 0; c < (ND == 3 ? W : 1); ++c) {
+                        double v = cw * S[0][a] * S[1][b];
+                        if constexpr (ND == 3) v *= S[2][c];
+                        unsafeAtomicAdd(&rho[lin(g, cl.G0[0] + o[0] - H + a, cl.G0[1] + o[1] - H + b,
+                                                 ND == 3 ? cl.G0[2] + o[2] - H + c : 0)], v);
+                    }
+            continue;
+        }
+        double *t = sR + (ND == 3 ? (o[0] * T + o[1]) * T + o[2] : o[0] * T + o[1]);
+#pragma unroll
+        for (int a = 0; a < W; ++a)
+#pragma unroll
+            for (int b = 0; b < W; ++b) {
+                const double v = cw * S[0][a] * S[1][b];
+                if constexpr (ND == 3) {
+#pragma unroll
+                    for (int c = 0; c < W; ++c) atomicAdd(&t[(a * T + b) * T + c], v * S[2][c]);
+                } else {
+                    atomicAdd(&t[a * T + b], v);
+                }
+            }
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < TN; t += blockDim.x) {
+        const double v = sR[t];
+        if (v == 0.) continue;
+        const int a = ND == 3 ? t / (T * T) : t / T, b = ND == 3 ? (t / T) % T : t % T, c = ND == 3 ? t % T : 0;
+        unsafeAtomicAdd(&rho[lin(g, cl.G0[0] - H + a, cl.G0[1] - H + b, ND == 3 ? cl.G0[2] - H + c : 0)], v);
+    }
 }
 
 // Global key of cell c (periodic indices in [0, N)): patch, 4^ND cluster,
@@ -380,16 +422,17 @@ void launch_ukin(const PartPtrs &A, const int32_t *perm, int64_t n, double *part
     SMI_LAUNCH_CHECK();
 }
 
-void launch_rho(const Geom &g, const SpeciesK &sp, const PartPtrs &A, const int32_t *perm, int64_t n, double *rho,
-                hipStream_t st)
+void launch_rho(const Geom &g, const SpeciesK &sp, const PartPtrs &A, const int32_t *perm, const int32_t *cell_off,
+                int64_t n, double *rho, hipStream_t st)
 {
     if (n == 0) return;
+    const dim3 grid(g.npatches * g.clpp);
     if (g.nd == 3 && g.order == 2)
-        hipLaunchKernelGGL((k_rho<3, 2>), dim3(nblk(n, 256)), dim3(256), 0, st, g, sp, A, perm, n, rho);
+        hipLaunchKernelGGL((k_rho<3, 2>), grid, dim3(256), 0, st, g, sp, A, perm, cell_off, rho);
     else if (g.nd == 3 && g.order == 4)
-        hipLaunchKernelGGL((k_rho<3, 4>), dim3(nblk(n, 256)), dim3(256), 0, st, g, sp, A, perm, n, rho);
+        hipLaunchKernelGGL((k_rho<3, 4>), grid, dim3(256), 0, st, g, sp, A, perm, cell_off, rho);
     else
-        hipLaunchKernelGGL((k_rho<2, 2>), dim3(nblk(n, 256)), dim3(256), 0, st, g, sp, A, perm, n, rho);
+        hipLaunchKernelGGL((k_rho<2, 2>), grid, dim3(128), 0, st, g, sp, A, perm, cell_off, rho);
     SMI_LAUNCH_CHECK();
 }
 

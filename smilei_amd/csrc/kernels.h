@@ -262,7 +262,7 @@ void launch_patch_counts_mixed(const Geom &g, const MixPtrs &M, const uint32_t *
 void launch_ukin_mixed(const MixPtrs &M, const int32_t *perm, int64_t n, double *partials, int nblocks,
                        hipStream_t st);
 void launch_rho_mixed(const Geom &g, const SpeciesKM &sp, const MixPtrs &M, const uint32_t *keys, const int32_t *perm,
-                      int64_t n, double *rho, hipStream_t st);
+                      const int32_t *cell_off, int64_t n, double *rho, hipStream_t st);
 
 // ---- initialisation (init.hip) ---------------------------------------
 // Particle i lives in cell cells[i/ppc] (or cell i/ppc when cells == null).
@@ -293,8 +293,9 @@ void launch_ukin(const PartPtrs &A, const int32_t *perm, int64_t n, double *part
                  hipStream_t st);
 // Sum of n weights (FP64 w or FP32 wf), per-block partials.
 void launch_wsum(const double *w, const float *wf, int64_t n, double *partials, int nblocks, hipStream_t st);
-void launch_rho(const Geom &g, const SpeciesK &sp, const PartPtrs &A, const int32_t *perm, int64_t n,
-                double *rho, hipStream_t st);
+// cell_off / perm as the sort left them (any cluster layout).
+void launch_rho(const Geom &g, const SpeciesK &sp, const PartPtrs &A, const int32_t *perm, const int32_t *cell_off,
+                int64_t n, double *rho, hipStream_t st);
 // Same density added in a fixed order (one thread per node gathering from
 // the sorted cells; cell_off / perm / lay as the sort left them).
 void launch_rho_gather(const Geom &g, const SpeciesK &sp, const PartPtrs &A, const int32_t *perm,

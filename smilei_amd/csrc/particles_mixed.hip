@@ -979,34 +979,56 @@ __global__ void k_ukin_mixed(MixPtrs M, const int32_t *__restrict__ perm, int64_
 }
 
 // Charge density of the mixed particles (FP64 accumulation): primal
-// stencil centred on the particle's node.
+// stencil centred on the particle's node.  One workgroup per cluster: its
+// particles' nodes are the cluster's 4^3, their stencils a tile of 4 + 2H
+// points per axis, summed with LDS atomics and flushed once (per-particle
+// global atomics: 21.2 ms for a 3.4e7-particle species at order 2, 8.46 ms
+// for 2.1e6 at order 4, against 0.69 and 0.20 ms).
 template <int ORDER>
-__global__ void k_rho_mixed(Geom g, SpeciesKM sp, MixPtrs M, const uint32_t *__restrict__ keys,
-                            const int32_t *__restrict__ perm, int64_t n, double *__restrict__ rho)
+__global__ void __launch_bounds__(256)
+k_rho_mixed(Geom g, SpeciesKM sp, MixPtrs M, const uint32_t *__restrict__ keys, const int32_t *__restrict__ perm,
+            const int32_t *__restrict__ cell_off, double *__restrict__ rho)
 {
-    constexpr int H = ORDER / 2, W = 2 * H + 1;
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= n) return;
-    const int i = perm[j];
-    int c[3];
-    node_of(g, keys[i] & kMask, c);
-    const float off[3] = {M.ox[i], M.oy[i], M.oz[i]};
-    double S[3][5];
-    int base[3];
-    for (int d = 0; d < 3; ++d) {
-        float w[5];
-        splinef<ORDER>(off[d], w);
-        for (int a = 0; a < W; ++a) S[d][a] = w[a];
-        base[d] = c[d] - H;
-    }
-    const double cwv = sp.cwd * (double)M.w[i];
-    for (int a = 0; a < W; ++a)
-        for (int b = 0; b < W; ++b)
-            for (int k = 0; k < W; ++k) {
-                const int64_t idx = ((int64_t)wrapi(base[0] + a, g.N[0]) * g.N[1] + wrapi(base[1] + b, g.N[1])) *
-                                        g.N[2] + wrapi(base[2] + k, g.N[2]);
-                unsafeAtomicAdd(&rho[idx], cwv * S[0][a] * S[1][b] * S[2][k]);
+    constexpr int H = ORDER / 2, W = 2 * H + 1, T = 4 + 2 * H, SY = T + 1, SX = T * SY;
+    __shared__ double sR[T * SX];
+    const Cl<1> cl = tile_of<1>(g, blockIdx.x);
+    const int s = cell_off[cl.gbase[0]], e = cell_off[cl.gbase[0] + 64];
+    if (s == e) return;  // uniform across the workgroup
+    for (int t = threadIdx.x; t < T * SX; t += blockDim.x) sR[t] = 0.;
+    __syncthreads();
+    for (int j = s + (int)threadIdx.x; j < e; j += blockDim.x) {
+        const int i = perm[j];
+        const int lc = (int)((int64_t)(keys[i] & kMask) - cl.gbase[0]);
+        if (lc < 0 || lc >= 64) continue;  // not in this cluster: corrupt state, flagged by the step
+        const float off[3] = {M.ox[i], M.oy[i], M.oz[i]};
+        double S[3][5];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            float w[5];
+            splinef<ORDER>(off[d], w);
+#pragma unroll
+            for (int a = 0; a < W; ++a) S[d][a] = w[a];
+        }
+        const double cwv = sp.cwd * (double)M.w[i];
+        double *t = sR + (lc >> 4) * SX + ((lc >> 2) & 3) * SY + (lc & 3);
+#pragma unroll
+        for (int a = 0; a < W; ++a)
+#pragma unroll
+            for (int b = 0; b < W; ++b) {
+                const double v = cwv * S[0][a] * S[1][b];
+#pragma unroll
+                for (int k = 0; k < W; ++k) atomicAdd(&t[a * SX + b * SY + k], v * S[2][k]);
             }
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < T * T * T; t += blockDim.x) {
+        const int a = t / (T * T), b = (t / T) % T, k = t % T;
+        const double v = sR[a * SX + b * SY + k];
+        if (v == 0.) continue;
+        const int idx = (wrapi(cl.G0[0] - H + a, g.N[0]) * g.N[1] + wrapi(cl.G0[1] - H + b, g.N[1])) * g.N[2] +
+                        wrapi(cl.G0[2] - H + k, g.N[2]);
+        unsafeAtomicAdd(&rho[idx], v);
+    }
 }
 
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
@@ -1141,13 +1163,14 @@ void launch_ukin_mixed(const MixPtrs &M, const int32_t *perm, int64_t n, double 
 }
 
 void launch_rho_mixed(const Geom &g, const SpeciesKM &sp, const MixPtrs &M, const uint32_t *keys, const int32_t *perm,
-                      int64_t n, double *rho, hipStream_t st)
+                      const int32_t *cell_off, int64_t n, double *rho, hipStream_t st)
 {
     if (n == 0) return;
+    const dim3 grid(g.npatches * g.clpp);
     if (g.order == 2)
-        hipLaunchKernelGGL(k_rho_mixed<2>, dim3(nblk(n, 256)), dim3(256), 0, st, g, sp, M, keys, perm, n, rho);
+        hipLaunchKernelGGL(k_rho_mixed<2>, grid, dim3(256), 0, st, g, sp, M, keys, perm, cell_off, rho);
     else
-        hipLaunchKernelGGL(k_rho_mixed<4>, dim3(nblk(n, 256)), dim3(256), 0, st, g, sp, M, keys, perm, n, rho);
+        hipLaunchKernelGGL(k_rho_mixed<4>, grid, dim3(256), 0, st, g, sp, M, keys, perm, cell_off, rho);
     SMI_LAUNCH_CHECK();
 }
 
