@@ -420,6 +420,53 @@ __device__ inline void esirkepov3d_win(const double (&S0)[3][ORDER + 2], const d
     (void)S;
 }
 
+// The same contributions with the transverse weight factorised,
+// W(b,c) = S0b (S0c + DSc/2) + DSb (S0c/2 + DSc/3), and the current factor in
+// the prefix sums along the current's axis: one FMA and one product per
+// column and one product per face, against eleven and two operations of the
+// reference's association, for sums whose order is free (tile atomics).  NT
+// window entries across the current, NA faces along it: NT = ORDER + 1, NA =
+// ORDER for a particle that keeps its node on every axis, NT = ORDER + 2,
+// NA = ORDER + 1 otherwise.  The face after the last window entry is left
+// out: its prefix sum is sum(DS) over the whole window, zero up to rounding.
+// add(c, i, j, k, value) as esirkepov3d_win.
+template <int ORDER, int NT, int NA, class Add>
+__device__ inline void esirkepov3d_fact(const double (&S0)[3][ORDER + 2], const double (&DS)[3][ORDER + 2],
+                                        const int *w0, const double *cr, Add add)
+{
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int bx = (c + 1) % 3, ex = (c + 2) % 3;
+        double P[NT], Q[NT], A[NA];
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            P[m] = fma(0.5, DS[ex][m], S0[ex][m]);
+            Q[m] = fma(kThird, DS[ex][m], 0.5 * S0[ex][m]);
+        }
+        double ps = DS[c][0];
+        A[0] = -cr[c] * ps;
+#pragma unroll
+        for (int r = 1; r < NA; ++r) {
+            ps += DS[c][r];
+            A[r] = -cr[c] * ps;
+        }
+#pragma unroll
+        for (int a = 0; a < NT; ++a)
+#pragma unroll
+            for (int b = 0; b < NT; ++b) {
+                const double t = fma(S0[bx][a], P[b], DS[bx][a] * Q[b]);
+#pragma unroll
+                for (int r = 1; r <= NA; ++r) {
+                    int idx[3];
+                    idx[c] = w0[c] + r;
+                    idx[bx] = w0[bx] + a;
+                    idx[ex] = w0[ex] + b;
+                    add(c, idx[0], idx[1], idx[2], A[r - 1] * t);
+                }
+            }
+    }
+}
+
 // 2D3V Esirkepov of Projector2D2Order::currents (Projector2D2Order.cpp:
 // 131-188): Jx prefix along x per column j, Jy prefix along y per row i,
 // Jz projected with the time-averaged shape.  add(c, i, j, v).
