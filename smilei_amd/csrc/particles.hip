@@ -31,8 +31,9 @@ namespace {
 using namespace dev;
 
 // Esirkepov currents of one 3D particle into the cluster's LDS tile: old
-// delta dold, new position in cell units pnn, old node ip; NT as
-// esirkepov3d_win.
+// delta dold, new position in cell units pnn, old node ip; NT / NT - 1 window
+// entries across / along the current (esirkepov3d_fact; NT = ORDER + 1: the
+// node is unchanged on every axis).
 template <int ORDER, int NT>
 __device__ inline void deposit3_tile(double *sJ, const Geom &g, const int *G0, const double *dold, const double *pnn,
                                      const int *ip, double cw)
@@ -42,16 +43,26 @@ __device__ inline void deposit3_tile(double *sJ, const Geom &g, const int *G0, c
     // J-tile strides: order-2 rows padded by one word (fp_cluster's layout)
     constexpr int JSY = ORDER == 2 ? JT + 1 : JT, JSX = JT * JSY, JSC = JT * JSX;
     double S0[3][ORDER + 2], DS[3][ORDER + 2];
-    int w0[3];
+    int w0[3] = {1, 1, 1};
 #pragma unroll
-    for (int d = 0; d < 3; ++d) esirkepov_window<ORDER>(dold[d], pnn[d], ip[d], S0[d], DS[d], w0[d]);
-    const double cr[3] = {cw * (g.dx[0] / g.dt), cw * (g.dx[1] / g.dt), cw * (g.dx[2] / g.dt)};
+    for (int d = 0; d < 3; ++d) {
+        if constexpr (NT == ORDER + 1) {
+            double s1[ORDER + 1];
+            spline<ORDER>(dold[d], S0[d]);
+            spline<ORDER>(pnn[d] - (double)ip[d], s1);
+#pragma unroll
+            for (int m = 0; m <= ORDER; ++m) DS[d][m] = s1[m] - S0[d][m];
+        } else {
+            esirkepov_window<ORDER>(dold[d], pnn[d], ip[d], S0[d], DS[d], w0[d]);
+        }
+    }
+    const double cr[3] = {cw * g.dxdt[0], cw * g.dxdt[1], cw * g.dxdt[2]};
     // tile coords of stencil index 0 along each axis
     const int o0 = ip[0] - (H + 1) - (G0[0] - TL::JO);
     const int o1 = ip[1] - (H + 1) - (G0[1] - TL::JO);
     const int o2 = ip[2] - (H + 1) - (G0[2] - TL::JO);
     double *sJb = sJ + o0 * JSX + o1 * JSY + o2;
-    esirkepov3d_win<ORDER, NT>(S0, DS, w0, cr, [&](int c, int a, int b, int k, double v) {
+    esirkepov3d_fact<ORDER, NT, NT - 1>(S0, DS, w0, cr, [&](int c, int a, int b, int k, double v) {
         atomicAdd(&sJb[c * JSC + a * JSX + b * JSY + k], v);
     });
 }
