@@ -152,14 +152,12 @@ bool want_placed(const smi_context *c)
     return c->p.deposit != SMI_DEPOSIT_DETERMINISTIC && !c->cell_order;
 }
 
-// Sort of species S from keys; tie: the kernel's recorded positions (the
-// step's sort) or null (the slots themselves: freshly loaded particles).
-void sort_species(smi_context *c, SpeciesState &S, const uint32_t *keys, bool counted, bool ordered,
-                  const int32_t *tie = nullptr)
+// Sort of freshly loaded particles of species S (ties: the slots themselves).
+void sort_loaded(smi_context *c, SpeciesState &S)
 {
-    if (!counted) S.mirrored = false;  // freshly loaded particles: one buffer holds them
+    S.mirrored = false;  // one buffer holds them
     S.lay = want_interleaved(c);
-    launch_sort(c->g, keys, S.n, S.sb, c->st, counted, ordered, S.lay, tie, counted && want_placed(c));
+    launch_sort(c->g, S.keys[c->cur], S.n, S.sb, c->st, false, true, S.lay, nullptr, false);
 }
 
 void drop_graphs(smi_context *c)
@@ -315,8 +313,7 @@ void enqueue_step(smi_context *c, bool timed)
     FieldSet f = c->fields();
     JPtrs J{f.J[0], f.J[1], f.J[2]};
     if (timed) SMI_HIP(hipEventRecord(c->ev[0], c->st));
-    if (!det)
-        for (int q = 0; q < 3; ++q) launch_fill(f.J[q], g.ncells, 0.0, c->st);  // restartRhoJ
+    if (!det) launch_clear_j(J, g.ncells, c->st);  // restartRhoJ
     enqueue_particles(c, a);
     if (timed) SMI_HIP(hipEventRecord(c->ev[1], c->st));
     if (det && !c->sp.empty()) {
@@ -328,9 +325,16 @@ void enqueue_step(smi_context *c, bool timed)
     launch_maxwell(g, f, c->st);
     if (timed) SMI_HIP(hipEventRecord(c->ev[3], c->st));
     const bool ordered = det || c->cell_order;
-    for (int id : c->moving) {
-        SpeciesState &s = c->sp[id];
-        sort_species(c, s, s.keys[1 - a], /*counted=*/true, ordered, want_rank(c) ? s.sb.rank : nullptr);
+    const int ns = (int)c->moving.size();
+    for (int g0 = 0; g0 < ns; g0 += kMaxMerged) {
+        SortTask tasks[kMaxMerged];
+        const int n = std::min(kMaxMerged, ns - g0);
+        for (int q = 0; q < n; ++q) {
+            SpeciesState &s = c->sp[c->moving[g0 + q]];
+            s.lay = want_interleaved(c);
+            tasks[q] = SortTask{s.keys[1 - a], s.n, &s.sb, want_rank(c) ? s.sb.rank : nullptr};
+        }
+        launch_sort(g, tasks, n, c->st, /*counted=*/true, ordered, want_interleaved(c), want_placed(c));
     }
     if (timed) SMI_HIP(hipEventRecord(c->ev[4], c->st));
 }
@@ -673,7 +677,7 @@ int smi_set_particles(smi_context *c, int s, int64_t n, const double *x, const d
         }
         launch_bin_initial(c->g, S.view(c->cur), n, S.keys[c->cur], c->st);
     }
-    sort_species(c, S, S.keys[c->cur], false, true);
+    sort_loaded(c, S);
     SMI_HIP(hipStreamSynchronize(c->st));
     return SMI_OK;
     SMI_CATCH
@@ -757,7 +761,7 @@ void init_particles(smi_context *c, int s, int64_t n, int ppc, const int32_t *d_
                 c->st);
     S.n = n;
     if (!c->mixed) launch_bin_initial(g, S.view(c->cur), n, S.keys[c->cur], c->st);
-    sort_species(c, S, S.keys[c->cur], false, true);
+    sort_loaded(c, S);
     SMI_HIP(hipStreamSynchronize(c->st));
 }
 
@@ -861,7 +865,7 @@ int smi_init_species_like(smi_context *c, int s, int src, double weight_scale, d
                      weight_scale, 0.0, mj.n ? mj.buf.p : nullptr, mj.n, drift_ux,
                      seed * 0x100000001B3ull + (uint64_t)s, c->st);
     S.n = R.n;
-    sort_species(c, S, S.keys[c->cur], false, true);
+    sort_loaded(c, S);
     SMI_HIP(hipStreamSynchronize(c->st));
     return SMI_OK;
     SMI_CATCH

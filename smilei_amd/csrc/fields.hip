@@ -122,6 +122,15 @@ __global__ void k_fill(double *p, int64_t n, double v)
     if (i < n) p[i] = v;
 }
 
+__global__ void k_clear_j(JPtrs J, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    J.Jx[i] = 0.;
+    J.Jy[i] = 0.;
+    J.Jz[i] = 0.;
+}
+
 __global__ void k_fill_i32(int32_t *p, int64_t n, int32_t v)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -383,6 +392,12 @@ void launch_fill(double *p, int64_t n, double v, hipStream_t st)
 {
     if (n <= 0) return;
     hipLaunchKernelGGL(k_fill, dim3(nblk(n, 256)), dim3(256), 0, st, p, n, v);
+    SMI_LAUNCH_CHECK();
+}
+
+void launch_clear_j(const JPtrs &J, int64_t n, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_clear_j, dim3(nblk(n, 256)), dim3(256), 0, st, J, n);
     SMI_LAUNCH_CHECK();
 }
 

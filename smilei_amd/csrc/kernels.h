@@ -206,6 +206,15 @@ int64_t sort_bsum_size(int64_t ncells);
 void launch_sort(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, hipStream_t st,
                  bool counted = false, bool in_cell_order = true, int layout = 0,
                  const int32_t *tie = nullptr, bool placed = false);
+// The same for up to kMaxMerged species in shared launches.
+struct SortTask {
+    const uint32_t *keys;
+    int64_t n;
+    SortBufs *sb;
+    const int32_t *tie;
+};
+void launch_sort(const Geom &g, const SortTask *tasks, int ns, hipStream_t st, bool counted, bool in_cell_order,
+                 int layout, bool placed);
 // Re-stores the current sorted order in another cluster layout (perm via
 // tmp); keys are those the order was sorted from.
 void launch_relayout(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, int from_layout,
@@ -284,6 +293,8 @@ struct FieldSet {
 // saveMagneticFields + MA + MF + centerMagneticFields on the periodic grid.
 void launch_maxwell(const Geom &g, const FieldSet &f, hipStream_t st);
 void launch_fill(double *p, int64_t n, double v, hipStream_t st);
+// Zero of the three components of J, one launch.
+void launch_clear_j(const JPtrs &J, int64_t n, hipStream_t st);
 void launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t st);
 // Diagnostics.
 // fids: the SMI_* component ids of the fields (their staggering).

@@ -23,6 +23,19 @@ namespace {
 
 constexpr uint32_t kKeyMask = (1u << 27) - 1;
 
+// One species of a sort launch; the species of a step share their launches
+// (blockIdx.y): small simulations are bound by the number of launches.
+struct SortOne {
+    const uint32_t *keys;
+    int64_t n;
+    const int32_t *tie;   // or null
+    int32_t *counts, *cell_off, *first, *perm, *tmp, *big, *nbig, *bsum, *clus_old;
+    uint8_t *stay;        // or null
+};
+struct SortSet {
+    SortOne s[kMaxMerged];
+};
+
 __global__ void k_hist(const uint32_t *__restrict__ keys, int64_t n, int32_t *__restrict__ counts)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -58,9 +71,10 @@ __device__ inline int block_exclusive_scan(int v, int &total)
     return base + incl - v;
 }
 
-__global__ void __launch_bounds__(kScanThreads)
-k_scan_reduce(const int32_t *__restrict__ in, int64_t n, int32_t *__restrict__ bsum)
+__global__ void __launch_bounds__(kScanThreads) k_scan_reduce(SortSet set, int64_t n)
 {
+    const int32_t *__restrict__ in = set.s[blockIdx.y].counts;
+    int32_t *__restrict__ bsum = set.s[blockIdx.y].bsum;
     const int64_t base = (int64_t)blockIdx.x * kScanTile;
     int s = 0;
 #pragma unroll
@@ -74,8 +88,9 @@ k_scan_reduce(const int32_t *__restrict__ in, int64_t n, int32_t *__restrict__ b
 }
 
 // Single-block exclusive scan of the block sums (in place).
-__global__ void __launch_bounds__(kScanThreads) k_scan_bsum(int32_t *__restrict__ bsum, int64_t nb)
+__global__ void __launch_bounds__(kScanThreads) k_scan_bsum(SortSet set, int64_t nb)
 {
+    int32_t *__restrict__ bsum = set.s[blockIdx.y].bsum;
     int carry = 0;
     for (int64_t b0 = 0; b0 < nb; b0 += kScanTile) {
         int v[kScanItems];
@@ -98,18 +113,52 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_bsum(int32_t *__restrict_
     }
 }
 
-// out[i] = bsum[block] + exclusive prefix inside the block; out[n] = total.
-// Each thread owns 16 consecutive entries, moved as four 16-byte vectors
-// (the entries of a full tile are 64-byte aligned); the ragged last tile
-// takes the scalar path.  stay (placed stayers, or null): in[i] -= stay[i]
-// after the totals are read, leaving the count of the bucket's atomic
-// places, and stay[i] = 0.  clus_old (or null): the previous out[] of every
-// cpcell-th entry (each cluster's first slot before this sort) is saved
-// there before it is overwritten.
-__global__ void __launch_bounds__(kScanThreads)
-k_scan_apply(int32_t *__restrict__ in, int64_t n, const int32_t *__restrict__ bsum, int32_t *__restrict__ out,
-             uint8_t *__restrict__ stay, int32_t *__restrict__ clus_old, int cpcell)
+// Where a block of k_scan_apply takes the sum of the tiles before its own
+// from: kPrefScanned, bsum scanned by k_scan_bsum; kPrefSums, the tile sums
+// of k_scan_reduce, added up by the block; kPrefCounts, the counts
+// themselves.  A block adds up to 2,048 sums (kPrefSums) or 32,768 counts
+// (kPrefCounts, eight L2 reads in flight per thread) in less time than the
+// launches it replaces take: the scan of 32^3 cells and two species takes
+// 10.6 us in one launch, 32.5 us in three per species.
+constexpr int kPrefScanned = 0, kPrefSums = 1, kPrefCounts = 2;
+constexpr int64_t kMaxPrefSums = 2048, kMaxPrefCounts = 8;  // tiles
+
+// out[i] = sum of the tiles before + exclusive prefix inside the block;
+// out[n] = total.  Each thread owns 16 consecutive entries, moved as four
+// 16-byte vectors (the entries of a full tile are 64-byte aligned); the
+// ragged last tile takes the scalar path.  stay (placed stayers, or null):
+// in[i] -= stay[i] after the totals are read, leaving the count of the
+// bucket's atomic places, and stay[i] = 0 (not with kPrefCounts: other blocks
+// still read in).  clus_old (or null): the previous out[] of every cpcell-th
+// entry (each cluster's first slot before this sort) is saved there before it
+// is overwritten.  Block 0 clears the work list of crowded cells.
+__global__ void __launch_bounds__(kScanThreads) k_scan_apply(SortSet set, int64_t n, int pref, int cpcell)
 {
+    const SortOne &S = set.s[blockIdx.y];
+    int32_t *__restrict__ in = S.counts;
+    int32_t *__restrict__ out = S.cell_off;
+    const int32_t *__restrict__ bsum = S.bsum;
+    uint8_t *__restrict__ stay = S.stay;
+    int32_t *__restrict__ clus_old = S.clus_old;
+    if (S.nbig && blockIdx.x == 0 && threadIdx.x < 2) S.nbig[threadIdx.x] = 0;
+    int before = 0;
+    if (pref == kPrefScanned) {
+        before = bsum[blockIdx.x];
+    } else {
+        int s = 0;
+        if (pref == kPrefSums) {
+            for (int i = threadIdx.x; i < (int)blockIdx.x; i += kScanThreads) s += bsum[i];
+        } else {
+            const int4 *src = reinterpret_cast<const int4 *>(in);
+            const int m = blockIdx.x * (kScanTile / 4);
+#pragma unroll 8
+            for (int i = threadIdx.x; i < m; i += kScanThreads) {
+                const int4 t = src[i];
+                s += (t.x + t.y) + (t.z + t.w);
+            }
+        }
+        block_exclusive_scan(s, before);
+    }
     const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
     const bool full = (int64_t)(blockIdx.x + 1) * kScanTile <= n;
     if (clus_old) {
@@ -136,7 +185,7 @@ k_scan_apply(int32_t *__restrict__ in, int64_t n, const int32_t *__restrict__ bs
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) s += v[k];
     int tot;
-    int ex = block_exclusive_scan(s, tot) + bsum[blockIdx.x];
+    int ex = block_exclusive_scan(s, tot) + before;
     int o[kScanItems];
 #pragma unroll
     for (int k = 0; k < kScanItems; ++k) {
@@ -201,12 +250,18 @@ k_scan_apply(int32_t *__restrict__ in, int64_t n, const int32_t *__restrict__ bs
 // 5.62).
 constexpr int kScatThreads = 256, kScatItems = 6, kScatTile = kScatThreads * kScatItems;
 
-__global__ void __launch_bounds__(kScatThreads)
-k_scatter(const uint32_t *__restrict__ keys, int64_t n, const int32_t *__restrict__ cell_off,
-          int32_t *__restrict__ counts, int32_t *__restrict__ perm, int cpc, int lay, int placed)
+__global__ void __launch_bounds__(kScatThreads) k_scatter(SortSet set, int cpc, int lay, int placed)
 {
+    const SortOne &S = set.s[blockIdx.y];
+    const uint32_t *__restrict__ keys = S.keys;
+    const int64_t n = S.n;
+    const int32_t *__restrict__ cell_off = S.cell_off;
+    int32_t *__restrict__ counts = S.counts;
+    int32_t *__restrict__ perm = S.first;
+    const int blocks = (int)((n + kScatTile - 1) / kScatTile);  // of this species; the grid is the largest's
+    if ((int)blockIdx.x >= blocks) return;
     const int lane = threadIdx.x & 63;
-    const int64_t i0 = (int64_t)dev::xcd_cluster(blockIdx.x, gridDim.x) * kScatTile +
+    const int64_t i0 = (int64_t)dev::xcd_cluster(blockIdx.x, blocks) * kScatTile +
                        (int64_t)(threadIdx.x >> 6) * (64 * kScatItems) + lane;
     uint32_t kk[kScatItems];
 #pragma unroll
@@ -246,18 +301,25 @@ k_scatter(const uint32_t *__restrict__ keys, int64_t n, const int32_t *__restric
 }
 
 // Canonical order inside a cell: by direction of motion, then source slot.
-// One thread per cell.  Buckets of up to kFixRegs particles are ranked in
-// registers (all loads issued together, rank = number of smaller
-// (direction, slot) pairs; the pairs are distinct because slots are);
-// buckets of up to kFixMid are left to k_bucket_fix_mid, larger ones go to
-// the work list `big` (count in nbig[0], appended by k_bucket_fix_mid) for
-// k_bucket_fix_big, or, without a list, to an insertion sort in memory.
+// One thread per cell, then one wavefront per crowded cell.  Buckets of up to
+// kFixRegs particles are ranked in registers (all loads issued together, rank
+// = number of smaller (direction, slot) pairs; the pairs are distinct because
+// slots are).  Each wavefront then runs those of its 64 cells that hold up to
+// kFixMid particles, two at a time where each fits in half of its lanes: a
+// lane's rank is counted against the keys of the cell's other lanes, read as
+// scalars.  2D plasma, 2.6e5 cells of 16 particles per species: 104 us per
+// species in two launches with one cell per wavefront at a time, 118 us
+// here for both.  Larger ones go to the work list `big` (count in
+// nbig[0]) for k_bucket_fix_big, or, without a list, to an insertion sort in
+// memory.  The stores of a cell follow the loads of all its places, so the
+// in-place case (dst == src) is safe.
 // The cell-major input is src; cpc == 0: sorted in place (dst == src);
 // cpc > 0: every particle is written to its lane-interleaved slot of the
 // cluster in dst.  The tie-break value of source slot v is tie[v] when tie
 // is given, else v.
 constexpr int kFixRegs = 16;
-constexpr int kFixMid = 64;
+constexpr int kFixMid = 256;
+constexpr int kFixPer = kFixMid / 64;
 
 // Where the tie-breaks come from: tie[v] (the cell-major position of slot
 // v in the previous sorted order, recorded by the particle kernel), or v
@@ -269,6 +331,11 @@ constexpr int kFixMid = 64;
 // motion is 13 (no patch face crossed) and its key need not be read either,
 // unless some axis is one cluster wide (a periodic wrap lands in the same
 // cluster): stay13 = 0 then.
+struct TieGeom {
+    int cpcell, ncl;
+    int lay;  // layout of the previous order's clusters
+    int stay13;
+};
 struct TieSrc {
     const int32_t *tie;
     const int32_t *clus_old;
@@ -276,6 +343,10 @@ struct TieSrc {
     int lay;  // layout of the previous order's clusters
     int64_t n;
     int stay13;
+    __device__ TieSrc(const SortOne &S, const TieGeom &G)
+        : tie(S.tie), clus_old(S.clus_old), cpcell(G.cpcell), ncl(G.ncl), lay(G.lay), n(S.n), stay13(G.stay13)
+    {
+    }
     // previous range [cs, cs + cn) of the cluster of cell g (cn = 0: none)
     __device__ void range(int64_t g, int &cs, int &cn) const
     {
@@ -303,73 +374,6 @@ __device__ inline uint64_t fix_key(const uint32_t *keys, const TieSrc &T, int32_
     return ((uint64_t)(keys[v] >> 27) << 32) | t;
 }
 
-__global__ void k_bucket_fix(const uint32_t *__restrict__ keys, int64_t ncells, const int32_t *__restrict__ cell_off,
-                             int32_t *src, int32_t *dst, int cpc, int lay, TieSrc T, int32_t *__restrict__ big,
-                             int32_t *__restrict__ nbig)
-{
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= ncells) return;
-    const int a = cell_off[g], b = cell_off[g + 1];
-    const int n = b - a;
-    int cs = 0, cn = 0;
-    if (cpc) {
-        const int64_t cb = g & ~(int64_t)(cpc - 1);
-        cs = cell_off[cb];
-        cn = cell_off[cb + cpc] - cs;
-    }
-    // final place of the particle of cell-major position pos
-    auto put = [&](int pos, int32_t v) { dst[cpc ? cs + layout_slot(lay, pos - cs, cn) : pos] = v; };
-    if (n < 2) {
-        if (cpc && n == 1) put(a, src[a]);
-        return;
-    }
-    int ocs, ocn;
-    T.range(g, ocs, ocn);
-    if (n <= kFixRegs) {
-        int32_t v[kFixRegs];
-        uint64_t k[kFixRegs];
-#pragma unroll
-        for (int i = 0; i < kFixRegs; ++i) v[i] = i < n ? src[a + i] : 0;
-#pragma unroll
-        for (int i = 0; i < kFixRegs; ++i) k[i] = i < n ? fix_key(keys, T, v[i], ocs, ocn) : ~0ull;
-        bool sorted = true;
-#pragma unroll
-        for (int i = 1; i < kFixRegs; ++i) sorted &= k[i - 1] < k[i] || i >= n;
-        if (sorted) {
-            if (cpc)
-#pragma unroll
-                for (int i = 0; i < kFixRegs; ++i)
-                    if (i < n) put(a + i, v[i]);
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < kFixRegs; ++i) {
-            int r = 0;
-#pragma unroll
-            for (int j = 0; j < kFixRegs; ++j) r += k[j] < k[i] ? 1 : 0;
-            if (i < n) put(a + r, v[i]);
-        }
-        return;
-    }
-    if (big) return;  // k_bucket_fix_mid, k_bucket_fix_big
-    int32_t *perm = src;
-    for (int i = a + 1; i < b; ++i) {
-        const int32_t v = perm[i];
-        const uint64_t kv = fix_key(keys, T, v, ocs, ocn);
-        int j = i - 1;
-        while (j >= a) {
-            const int32_t u = perm[j];
-            const uint64_t ku = fix_key(keys, T, u, ocs, ocn);
-            if (ku <= kv) break;
-            perm[j + 1] = u;
-            --j;
-        }
-        perm[j + 1] = v;
-    }
-    if (cpc)
-        for (int i = a; i < b; ++i) put(i, perm[i]);
-}
-
 // Wave-aggregated append of the lanes with `want` to a counter: returns
 // each such lane's index (one atomic per wavefront).
 __device__ inline int wave_append(bool want, int32_t *counter)
@@ -384,42 +388,150 @@ __device__ inline int wave_append(bool want, int32_t *counter)
     return base + __popcll(m & ((1ull << lane) - 1));
 }
 
-// Each wavefront scans 64 consecutive cells and runs those with kFixRegs <
-// n <= kFixMid particles one after the other, with the whole wavefront:
-// lane l holds place l, its rank = the number of smaller keys over the
-// wavefront (shuffles).  The stores follow the loads of every lane, so the
-// in-place case is safe.  Cells with more particles go to the work list
-// `big` for k_bucket_fix_big.
-__global__ void __launch_bounds__(256)
-k_bucket_fix_mid(const uint32_t *__restrict__ keys, int64_t ncells, const int32_t *__restrict__ cell_off,
-                 int32_t *src, int32_t *dst, int cpc, int lay, TieSrc T, int32_t *__restrict__ big,
-                 int32_t *__restrict__ nbig)
+// Key of lane j (the same j for all lanes).
+__device__ inline uint64_t lane_key(uint64_t k, int j)
 {
+    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)k, j), hi = __builtin_amdgcn_readlane((uint32_t)(k >> 32), j);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+__global__ void __launch_bounds__(256) k_bucket_fix(SortSet set, int64_t ncells, int cpc, int lay, TieGeom G)
+{
+    const SortOne &S = set.s[blockIdx.y];
+    const uint32_t *__restrict__ keys = S.keys;
+    const int32_t *__restrict__ cell_off = S.cell_off;
+    int32_t *src = S.first, *dst = S.perm;
+    const TieSrc T(S, G);
     const int lane = threadIdx.x & 63;
-    const int64_t g0 = (int64_t)blockIdx.x * blockDim.x + (threadIdx.x & ~63);
-    const int64_t gl = g0 + lane;
-    const int nl = gl < ncells ? cell_off[gl + 1] - cell_off[gl] : 0;
-    const int ib = wave_append(nl > kFixMid, &nbig[0]);
-    if (nl > kFixMid) big[ib] = (int32_t)gl;
-    uint64_t todo = __ballot(nl > kFixRegs && nl <= kFixMid);
-    while (todo) {
-        const int bit = __ffsll((unsigned long long)todo) - 1;
-        todo &= todo - 1;
-        const int64_t g = g0 + bit;
-        const int a = cell_off[g], n = cell_off[g + 1] - a;
-        int cs = 0, cn = 0;
-        if (cpc) {
-            const int64_t cb = g & ~(int64_t)(cpc - 1);
-            cs = cell_off[cb];
-            cn = cell_off[cb + cpc] - cs;
+    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = g < ncells ? cell_off[g] : 0, b = g < ncells ? cell_off[g + 1] : 0;
+    const int n = b - a;
+    // final place of the particle of cell-major position pos of cell gc
+    auto cluster = [&](int64_t gc, int &cs, int &cn) {
+        cs = 0;
+        cn = 0;
+        if (!cpc) return;
+        const int64_t cb = gc & ~(int64_t)(cpc - 1);
+        cs = cell_off[cb];
+        cn = cell_off[cb + cpc] - cs;
+    };
+    if (n > 0 && n <= kFixRegs) {
+        int cs, cn;
+        cluster(g, cs, cn);
+        auto put = [&](int pos, int32_t v) { dst[cpc ? cs + layout_slot(lay, pos - cs, cn) : pos] = v; };
+        if (n == 1) {
+            if (cpc) put(a, src[a]);
+        } else {
+            int ocs, ocn;
+            T.range(g, ocs, ocn);
+            int32_t v[kFixRegs];
+            uint64_t k[kFixRegs];
+#pragma unroll
+            for (int i = 0; i < kFixRegs; ++i) v[i] = i < n ? src[a + i] : 0;
+#pragma unroll
+            for (int i = 0; i < kFixRegs; ++i) k[i] = i < n ? fix_key(keys, T, v[i], ocs, ocn) : ~0ull;
+            bool sorted = true;
+#pragma unroll
+            for (int i = 1; i < kFixRegs; ++i) sorted &= k[i - 1] < k[i] || i >= n;
+            if (sorted) {
+                if (cpc)
+#pragma unroll
+                    for (int i = 0; i < kFixRegs; ++i)
+                        if (i < n) put(a + i, v[i]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < kFixRegs; ++i) {
+                    int r = 0;
+#pragma unroll
+                    for (int j = 0; j < kFixRegs; ++j) r += k[j] < k[i] ? 1 : 0;
+                    if (i < n) put(a + r, v[i]);
+                }
+            }
         }
-        int ocs, ocn;
+    }
+    if (!S.big) {
+        if (n <= kFixRegs) return;
+        int cs, cn, ocs, ocn;
+        cluster(g, cs, cn);
         T.range(g, ocs, ocn);
-        const int32_t v = lane < n ? src[a + lane] : 0;
-        const uint64_t k = lane < n ? fix_key(keys, T, v, ocs, ocn) : ~0ull;
+        int32_t *perm = src;
+        for (int i = a + 1; i < b; ++i) {
+            const int32_t v = perm[i];
+            const uint64_t kv = fix_key(keys, T, v, ocs, ocn);
+            int j = i - 1;
+            while (j >= a) {
+                const int32_t u = perm[j];
+                const uint64_t ku = fix_key(keys, T, u, ocs, ocn);
+                if (ku <= kv) break;
+                perm[j + 1] = u;
+                --j;
+            }
+            perm[j + 1] = v;
+        }
+        if (cpc)
+            for (int i = a; i < b; ++i) dst[cs + layout_slot(lay, i - cs, cn)] = perm[i];
+        return;
+    }
+    const int ib = wave_append(n > kFixMid, &S.nbig[0]);
+    if (n > kFixMid) S.big[ib] = (int32_t)g;
+    // crowded cells of this wavefront's 64: pairs of up to 32 particles
+    const int64_t g0 = g - lane;
+    uint64_t half = __ballot(n > kFixRegs && n <= 32);
+    while (half) {
+        const int first = __ffsll((unsigned long long)half) - 1;
+        half &= half - 1;
+        const int second = half ? __ffsll((unsigned long long)half) - 1 : -1;
+        half &= half - 1;
+        const int mine = lane >= 32 ? second : first;  // this lane's cell, -1: none
+        const int l = lane & 31;
+        const int64_t gm = g0 + (mine < 0 ? first : mine);
+        const int am = cell_off[gm], nm = mine < 0 ? 0 : cell_off[gm + 1] - am;
+        int cs, cn, ocs, ocn;
+        cluster(gm, cs, cn);
+        T.range(gm, ocs, ocn);
+        const int32_t v = l < nm ? src[am + l] : 0;
+        const uint64_t k = l < nm ? fix_key(keys, T, v, ocs, ocn) : ~0ull;
+        const int n0 = __builtin_amdgcn_readlane(nm, 0), n1 = __builtin_amdgcn_readlane(nm, 32);
+        const int most = n0 > n1 ? n0 : n1;
         int r = 0;
-        for (int j = 0; j < n; ++j) r += __shfl(k, j, 64) < k ? 1 : 0;
-        if (lane < n) dst[cpc ? cs + layout_slot(lay, a + r - cs, cn) : a + r] = v;
+        for (int j = 0; j < most; ++j) {  // places past a cell's end hold the largest key: never smaller
+            const uint64_t k0 = lane_key(k, j), k1 = lane_key(k, 32 + j);
+            r += (lane < 32 ? k0 : k1) < k ? 1 : 0;
+        }
+        if (l < nm) dst[cpc ? cs + layout_slot(lay, am + r - cs, cn) : am + r] = v;
+    }
+    // and the others, up to kFixPer places per lane
+    uint64_t whole = __ballot(n > 32 && n <= kFixMid);
+    while (whole) {
+        const int64_t gm = g0 + (__ffsll((unsigned long long)whole) - 1);
+        whole &= whole - 1;
+        const int am = cell_off[gm], nm = __builtin_amdgcn_readfirstlane(cell_off[gm + 1] - am);
+        int cs, cn, ocs, ocn;
+        cluster(gm, cs, cn);
+        T.range(gm, ocs, ocn);
+        int32_t v[kFixPer];
+        uint64_t k[kFixPer];
+        int r[kFixPer];
+#pragma unroll
+        for (int q = 0; q < kFixPer; ++q) {
+            const int l = lane + 64 * q;
+            r[q] = 0;
+            v[q] = l < nm ? src[am + l] : 0;
+        }
+#pragma unroll
+        for (int q = 0; q < kFixPer; ++q) k[q] = lane + 64 * q < nm ? fix_key(keys, T, v[q], ocs, ocn) : ~0ull;
+#pragma unroll
+        for (int q = 0; q < kFixPer; ++q) {
+            const int end = nm - 64 * q < 64 ? nm - 64 * q : 64;
+            for (int j = 0; j < end; ++j) {
+                const uint64_t kj = lane_key(k[q], j);
+#pragma unroll
+                for (int m = 0; m < kFixPer; ++m) r[m] += kj < k[m] ? 1 : 0;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kFixPer; ++q)
+            if (lane + 64 * q < nm) dst[cpc ? cs + layout_slot(lay, am + r[q] - cs, cn) : am + r[q]] = v[q];
     }
 }
 
@@ -436,11 +548,25 @@ constexpr int kBigLds = 4096;
 constexpr int kBigPer = kBigLds / kBigThreads;
 constexpr int kBigBlocks = 1024;
 
-__global__ void __launch_bounds__(kBigThreads)
-k_bucket_fix_big(const uint32_t *__restrict__ keys, const int32_t *__restrict__ cell_off, int32_t *src, int32_t *dst,
-                 int32_t *scr, int cpc, int lay, TieSrc T, const int32_t *__restrict__ big,
-                 int32_t *__restrict__ nbig)
+// Workgroups for the crowded cells of n particles: there are at most n / 257
+// such cells and usually none, and a workgroup that finds the list empty still
+// costs its dispatch (1,024 of them, with 48 KB of LDS each: 13 us per
+// species).  All 1,024 only where the mean cell is half way to crowded.
+inline unsigned big_blocks(int64_t n, int64_t ncells)
 {
+    const int64_t b = (n + 2047) / 2048, most = n > ncells * (kFixMid / 2) ? kBigBlocks : 192;
+    return (unsigned)(b < most ? b : most);
+}
+
+__global__ void __launch_bounds__(kBigThreads) k_bucket_fix_big(SortSet set, int cpc, int lay, TieGeom G)
+{
+    const SortOne &S = set.s[blockIdx.y];
+    const uint32_t *__restrict__ keys = S.keys;
+    const int32_t *__restrict__ cell_off = S.cell_off;
+    int32_t *src = S.first, *dst = S.perm, *scr = S.tmp;
+    const TieSrc T(S, G);
+    const int32_t *__restrict__ big = S.big;
+    int32_t *__restrict__ nbig = S.nbig;
     __shared__ uint64_t sK[kBigLds];
     __shared__ int32_t sV[kBigLds];
     __shared__ int sItem;
@@ -577,57 +703,80 @@ inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 int64_t sort_bsum_size(int64_t ncells) { return (ncells + kScanTile - 1) / kScanTile + 1; }
 
-void launch_sort(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, hipStream_t st, bool counted,
-                 bool in_cell_order, int layout, const int32_t *tie, bool placed)
+void launch_sort(const Geom &g, const SortTask *tasks, int ns, hipStream_t st, bool counted, bool in_cell_order,
+                 int layout, bool placed)
 {
+    if (ns < 1 || ns > kMaxMerged) throw Error(-1, "bad species count of a sort launch");
     placed = placed && counted && !in_cell_order;
     const int64_t nc = g.ncells;
-    if (n > 0 && !counted) {
-        hipLaunchKernelGGL(k_hist, dim3(nblk(n, 256)), dim3(256), 0, st, keys, n, sb.counts);
-        SMI_LAUNCH_CHECK();
-    }
-    const int64_t nb = (nc + kScanTile - 1) / kScanTile;
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(kScanThreads), 0, st, (const int32_t *)sb.counts, nc,
-                       sb.bsum);
-    SMI_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_scan_bsum, dim3(1), dim3(kScanThreads), 0, st, sb.bsum, nb);
-    SMI_LAUNCH_CHECK();
     // the in-cell pass of the step's sort computes the ties of the particles
     // that stayed in their cluster from the clusters' previous ranges
     int stay13 = 1;
     for (int d = 0; d < g.nd; ++d)
         if (g.npatch[d] * g.n[d] <= 4) stay13 = 0;
-    const TieSrc T{tie, counted && tie && in_cell_order ? sb.clus_old : nullptr, g.cells_per_cl,
-                   (int)(nc / g.cells_per_cl), layout, n, stay13};
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(kScanThreads), 0, st, sb.counts, nc,
-                       (const int32_t *)sb.bsum, sb.cell_off, placed ? sb.stay : nullptr,
-                       const_cast<int32_t *>(T.clus_old), g.cells_per_cl);
-    SMI_LAUNCH_CHECK();
-    if (n > 0) {
-        // cell-major places go straight to perm unless the canonical order
-        // inside the cells and the interleaved layout are both asked for:
-        // then they are ordered in tmp and laid out into perm
-        const int cpc = layout ? g.cells_per_cl : 0;
-        int32_t *first = in_cell_order && layout ? sb.tmp : sb.perm;
-        hipLaunchKernelGGL(k_scatter, dim3(nblk(n, kScatTile)), dim3(kScatThreads), 0, st, keys, n, (const int32_t *)sb.cell_off,
-                           sb.counts, first, in_cell_order ? 0 : cpc, layout, placed ? 1 : 0);
-        SMI_LAUNCH_CHECK();
-        if (in_cell_order) {
-            if (sb.big) launch_fill_i32(sb.nbig, 2, 0, st);
-            hipLaunchKernelGGL(k_bucket_fix, dim3(nblk(nc, 256)), dim3(256), 0, st, keys, nc,
-                               (const int32_t *)sb.cell_off, first, sb.perm, cpc, layout, T, sb.big, sb.nbig);
+    const TieGeom G{g.cells_per_cl, (int)(nc / g.cells_per_cl), layout, stay13};
+    // cell-major places go straight to perm unless the canonical order inside
+    // the cells and the interleaved layout are both asked for: then they are
+    // ordered in tmp and laid out into perm
+    const int cpc = layout ? g.cells_per_cl : 0;
+    SortSet set{};
+    int64_t most = 0;
+    bool big = false;
+    for (int q = 0; q < ns; ++q) {
+        const SortTask &t = tasks[q];
+        const SortBufs &sb = *t.sb;
+        SortOne &S = set.s[q];
+        S.keys = t.keys;
+        S.n = t.n;
+        S.tie = t.tie;
+        S.counts = sb.counts;
+        S.cell_off = sb.cell_off;
+        S.first = in_cell_order && layout ? sb.tmp : sb.perm;
+        S.perm = sb.perm;
+        S.tmp = sb.tmp;
+        S.big = sb.big;
+        S.nbig = in_cell_order ? sb.nbig : nullptr;
+        S.bsum = sb.bsum;
+        S.clus_old = counted && t.tie && in_cell_order ? sb.clus_old : nullptr;
+        S.stay = placed ? sb.stay : nullptr;
+        most = t.n > most ? t.n : most;
+        big |= sb.big != nullptr;
+        if (t.n > 0 && !counted) {
+            hipLaunchKernelGGL(k_hist, dim3(nblk(t.n, 256)), dim3(256), 0, st, t.keys, t.n, sb.counts);
             SMI_LAUNCH_CHECK();
-            if (sb.big) {
-                hipLaunchKernelGGL(k_bucket_fix_mid, dim3(nblk(nc, 256)), dim3(256), 0, st, keys, nc,
-                                   (const int32_t *)sb.cell_off, first, sb.perm, cpc, layout, T, sb.big, sb.nbig);
-                SMI_LAUNCH_CHECK();
-                hipLaunchKernelGGL(k_bucket_fix_big, dim3(kBigBlocks), dim3(kBigThreads), 0, st, keys,
-                                   (const int32_t *)sb.cell_off, first, sb.perm, sb.tmp, cpc, layout, T,
-                                   (const int32_t *)sb.big, sb.nbig);
-                SMI_LAUNCH_CHECK();
-            }
         }
     }
+    const int64_t nb = (nc + kScanTile - 1) / kScanTile;
+    const int pref = nb <= kMaxPrefCounts && !placed ? kPrefCounts : (nb <= kMaxPrefSums ? kPrefSums : kPrefScanned);
+    const dim3 tiles((unsigned)nb, ns);
+    if (pref != kPrefCounts) {
+        hipLaunchKernelGGL(k_scan_reduce, tiles, dim3(kScanThreads), 0, st, set, nc);
+        SMI_LAUNCH_CHECK();
+    }
+    if (pref == kPrefScanned) {
+        hipLaunchKernelGGL(k_scan_bsum, dim3(1, ns), dim3(kScanThreads), 0, st, set, nb);
+        SMI_LAUNCH_CHECK();
+    }
+    hipLaunchKernelGGL(k_scan_apply, tiles, dim3(kScanThreads), 0, st, set, nc, pref, g.cells_per_cl);
+    SMI_LAUNCH_CHECK();
+    if (most == 0) return;
+    hipLaunchKernelGGL(k_scatter, dim3(nblk(most, kScatTile), ns), dim3(kScatThreads), 0, st, set,
+                       in_cell_order ? 0 : cpc, layout, placed ? 1 : 0);
+    SMI_LAUNCH_CHECK();
+    if (!in_cell_order) return;
+    hipLaunchKernelGGL(k_bucket_fix, dim3(nblk(nc, 256), ns), dim3(256), 0, st, set, nc, cpc, layout, G);
+    SMI_LAUNCH_CHECK();
+    if (big) {
+        hipLaunchKernelGGL(k_bucket_fix_big, dim3(big_blocks(most, nc), ns), dim3(kBigThreads), 0, st, set, cpc, layout, G);
+        SMI_LAUNCH_CHECK();
+    }
+}
+
+void launch_sort(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, hipStream_t st, bool counted,
+                 bool in_cell_order, int layout, const int32_t *tie, bool placed)
+{
+    const SortTask one{keys, n, &sb, tie};
+    launch_sort(g, &one, 1, st, counted, in_cell_order, layout, placed);
 }
 
 void launch_relayout(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, int from_layout,
