@@ -232,13 +232,10 @@ __global__ void __launch_bounds__(256) k_bin_count(Proj3Args a, Bins b)
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
     const int key = i < a.n ? node_bin<ORDER>(a, b, i) : -1;
-    const int before = __shfl_up(key, 1, 64);
-    const uint64_t heads = __ballot(lane == 0 || before != key);
-    const int head = 63 - __clzll((unsigned long long)(heads & (lane == 63 ? ~0ull : ((2ull << lane) - 1))));
-    const uint64_t above = head == 63 ? 0ull : heads & (~0ull << (head + 1));
-    const int next = above ? __ffsll((unsigned long long)above) - 1 : 64;
+    int head, len;
+    key_run((uint32_t)key, head, len);
     int first = 0;
-    if (lane == head && key >= 0) first = atomicAdd(&b.count[key], next - head);
+    if (lane == head && key >= 0) first = atomicAdd(&b.count[key], len);
     first = __shfl(first, head, 64);
     if (i < a.n) {
         b.key[i] = key;

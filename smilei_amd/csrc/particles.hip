@@ -621,49 +621,48 @@ __global__ void __launch_bounds__(64) k_det_deposit2(Geom g, const DetSpecies *_
 
 // Ghost sum along dimension d for the three components:
 // low[n + a] += this[a]; this[a] = low[n + a], a in [0, 1 + 2*os + dual).
-__global__ void k_ghost_sum(Geom g, int d, double *__restrict__ pj)
+// The component is the workgroup's (blockIdx.y), the patch too (`blocks` of
+// them per slab), so that extents and offsets are scalars: picked per thread
+// they were arrays in scratch memory, 18 us a pass over 8 patches of 32^3
+// cells against 5.5.
+__global__ void __launch_bounds__(256) k_ghost_sum(Geom g, int d, int blocks, double *__restrict__ pj)
 {
-    const PJLayout L = pj_layout(g);
-    int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    // enumerate (patch, component, point in the plane slab)
-    int64_t slab[3];
-    for (int c = 0; c < 3; ++c) {
-        const int gsp = 1 + 2 * g.os + (c == d ? 1 : 0);
+    const int c = blockIdx.y, p = blockIdx.x / blocks;
+    int r = (int)(blockIdx.x - p * blocks) * 256 + threadIdx.x;
+    int np[3], dm[3], ext[3];
+    int64_t off = 0, per = 0;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        np[e] = e < g.nd ? g.n[e] + 2 * g.os + 1 : 1;
+        dm[e] = np[e] + (e == c && e < g.nd ? 1 : 0);
+        ext[e] = e == d ? 1 + 2 * g.os + (c == d ? 1 : 0) : dm[e];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
         int64_t sz = 1;
-        for (int e = 0; e < 3; ++e) sz *= (e == d ? gsp : L.dims[c][e]);
-        slab[c] = sz;
+#pragma unroll
+        for (int e = 0; e < 3; ++e) sz *= np[e] + (e == q && e < g.nd ? 1 : 0);
+        if (q < c) off += sz;
+        per += sz;
     }
-    const int64_t per_patch = slab[0] + slab[1] + slab[2];
-    if (t >= per_patch * g.npatches) return;
-    const int p = (int)(t / per_patch);
-    int64_t r = t % per_patch;
-    int c = 0;
-    while (r >= slab[c]) {
-        r -= slab[c];
-        ++c;
-    }
-    const int gsp = 1 + 2 * g.os + (c == d ? 1 : 0);
-    int ext[3];
-    for (int e = 0; e < 3; ++e) ext[e] = e == d ? gsp : L.dims[c][e];
-    int idx[3];
-    idx[2] = (int)(r % ext[2]);
-    idx[1] = (int)((r / ext[2]) % ext[1]);
-    idx[0] = (int)(r / ((int64_t)ext[2] * ext[1]));
-    int pc[3];
-    pc[0] = p / (g.npatch[1] * g.npatch[2]);
-    pc[1] = (p / g.npatch[2]) % g.npatch[1];
-    pc[2] = p % g.npatch[2];
-    pc[d] = wrapi(pc[d] - 1, g.npatch[d]);
+    const int row = ext[1] * ext[2];
+    const int i = r / row;
+    if (i >= ext[0]) return;
+    r -= i * row;
+    const int j = r / ext[2], k = r - j * ext[2];
+    int pc[3] = {p / (g.npatch[1] * g.npatch[2]), (p / g.npatch[2]) % g.npatch[1], p % g.npatch[2]};
+#pragma unroll
+    for (int e = 0; e < 3; ++e)
+        if (e == d) pc[e] = wrapi(pc[e] - 1, g.npatch[e]);
     const int lp = (pc[0] * g.npatch[1] + pc[1]) * g.npatch[2] + pc[2];
-    const int *dm = L.dims[c];
-    double *me = pj + (int64_t)p * L.per + L.off[c];
-    double *lo = pj + (int64_t)lp * L.per + L.off[c];
-    int li[3] = {idx[0], idx[1], idx[2]};
-    li[d] += g.n[d];
-    const int64_t a = ((int64_t)li[0] * dm[1] + li[1]) * dm[2] + li[2];
-    const int64_t b = ((int64_t)idx[0] * dm[1] + idx[1]) * dm[2] + idx[2];
-    lo[a] += me[b];
-    me[b] = lo[a];
+    const int64_t b = ((int64_t)i * dm[1] + j) * dm[2] + k;
+    const int64_t step = d == 0 ? (int64_t)dm[1] * dm[2] : (d == 1 ? dm[2] : 1);
+    const int nd = d == 0 ? g.n[0] : (d == 1 ? g.n[1] : g.n[2]);
+    double *me = pj + p * per + off, *lo = pj + lp * per + off;
+    const int64_t a = b + nd * step;
+    const double sum = lo[a] + me[b];
+    lo[a] = sum;
+    me[b] = sum;
 }
 
 // Global J[g] = owning patch's ghost-summed value.
@@ -780,15 +779,16 @@ void launch_ghost_sum(const Geom &g, double *pj, hipStream_t st)
 {
     const PJLayout L = pj_layout(g);
     for (int d = 0; d < g.nd; ++d) {
-        int64_t per = 0;
+        int64_t slab = 0;  // the largest component's
         for (int c = 0; c < 3; ++c) {
             const int gsp = 1 + 2 * g.os + (c == d ? 1 : 0);
             int64_t sz = 1;
             for (int e = 0; e < 3; ++e) sz *= (e == d ? gsp : L.dims[c][e]);
-            per += sz;
+            slab = sz > slab ? sz : slab;
         }
-        const int64_t tot = per * g.npatches;
-        hipLaunchKernelGGL(k_ghost_sum, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, g, d, pj);
+        const int64_t blocks = (slab + 255) / 256;
+        hipLaunchKernelGGL(k_ghost_sum, dim3((unsigned)(blocks * g.npatches), 3), dim3(256), 0, st, g, d, (int)blocks,
+                           pj);
         SMI_LAUNCH_CHECK();
     }
 }

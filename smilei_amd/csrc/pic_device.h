@@ -120,6 +120,19 @@ __device__ inline void split_node(double xn, int N, int &node, float &off)
     off = f;
 }
 
+// Run of neighbouring lanes with this lane's key: its first lane and length.
+// Particles in cell order have long runs, which then share one atomic.  Every
+// lane of the wavefront calls it.
+__device__ inline void key_run(uint32_t key, int &head, int &len)
+{
+    const int lane = threadIdx.x & 63;
+    const uint32_t before = __shfl_up(key, 1, 64);
+    const uint64_t heads = __ballot(lane == 0 || before != key);
+    head = 63 - __clzll((unsigned long long)(heads & (lane == 63 ? ~0ull : ((2ull << lane) - 1))));
+    const uint64_t above = head == 63 ? 0ull : heads & (~0ull << (head + 1));
+    len = (above ? __ffsll((unsigned long long)above) - 1 : 64) - head;
+}
+
 // In-patch cell key (Cluster3D::CellKey, nvidiaParticles.cu:639-660) of a
 // position inside patch `pc`; clamped against rounding at the upper face.
 template <int ND>
@@ -139,6 +152,33 @@ __device__ inline int32_t cell_key(const Geom &g, const int *pc, const double *x
         const int cl = (ic[0] >> 2) * g.ncl[1] + (ic[1] >> 2);
         return cl * 16 + 4 * (ic[0] & 3) + (ic[1] & 3);
     }
+}
+
+// Global cell key (patch, then in-patch key) of a position in the box, the
+// patch as Patch::initStep3's limits put it.
+template <int ND>
+__device__ inline uint32_t position_key(const Geom &g, const double *x)
+{
+    int pc[3] = {0, 0, 0}, ic[3] = {0, 0, 0};
+    for (int d = 0; d < ND; ++d) {
+        int c = (int)floor(x[d] / g.plen[d]);
+        c = c < 0 ? 0 : (c > g.npatch[d] - 1 ? g.npatch[d] - 1 : c);
+        while (c > 0 && x[d] < (double)c * g.plen[d]) --c;
+        while (c < g.npatch[d] - 1 && x[d] >= (double)(c + 1) * g.plen[d]) ++c;
+        pc[d] = c;
+        int k = (int)floor(x[d] * (1.0 / g.dx[d])) - c * g.n[d];
+        ic[d] = k < 0 ? 0 : (k > g.n[d] - 1 ? g.n[d] - 1 : k);
+    }
+    int key;
+    if constexpr (ND == 3) {
+        const int cl = ((ic[0] >> 2) * g.ncl[1] + (ic[1] >> 2)) * g.ncl[2] + (ic[2] >> 2);
+        key = cl * 64 + 16 * (ic[0] & 3) + 4 * (ic[1] & 3) + (ic[2] & 3);
+    } else {
+        const int cl = (ic[0] >> 2) * g.ncl[1] + (ic[1] >> 2);
+        key = cl * 16 + 4 * (ic[0] & 3) + (ic[1] & 3);
+    }
+    const int p = (pc[0] * g.npatch[1] + pc[1]) * g.npatch[2] + pc[2];
+    return (uint32_t)((int64_t)p * g.cpp + key);
 }
 
 // Boris push (PusherBoris.cpp:80-127), FP64, reference association order.

@@ -39,8 +39,10 @@ struct SortSet {
 __global__ void k_hist(const uint32_t *__restrict__ keys, int64_t n, int32_t *__restrict__ counts)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    atomicAdd(&counts[keys[i] & kKeyMask], 1);
+    const uint32_t key = i < n ? keys[i] & kKeyMask : ~0u;
+    int head, len;
+    dev::key_run(key, head, len);
+    if ((int)(threadIdx.x & 63) == head && i < n) atomicAdd(&counts[key], len);
 }
 
 constexpr int kScanThreads = 256;
@@ -675,26 +677,7 @@ __global__ void k_bin_initial(Geom g, PartPtrs A, int64_t n, uint32_t *__restric
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const double x[3] = {A.x[i], A.y[i], ND == 3 ? A.z[i] : 0.};
-    int pc[3] = {0, 0, 0}, ic[3] = {0, 0, 0};
-    for (int d = 0; d < ND; ++d) {
-        int c = (int)floor(x[d] / g.plen[d]);
-        c = c < 0 ? 0 : (c > g.npatch[d] - 1 ? g.npatch[d] - 1 : c);
-        while (c > 0 && x[d] < (double)c * g.plen[d]) --c;
-        while (c < g.npatch[d] - 1 && x[d] >= (double)(c + 1) * g.plen[d]) ++c;
-        pc[d] = c;
-        int k = (int)floor(x[d] * (1.0 / g.dx[d])) - c * g.n[d];
-        ic[d] = k < 0 ? 0 : (k > g.n[d] - 1 ? g.n[d] - 1 : k);
-    }
-    int key;
-    if constexpr (ND == 3) {
-        const int cl = ((ic[0] >> 2) * g.ncl[1] + (ic[1] >> 2)) * g.ncl[2] + (ic[2] >> 2);
-        key = cl * 64 + 16 * (ic[0] & 3) + 4 * (ic[1] & 3) + (ic[2] & 3);
-    } else {
-        const int cl = (ic[0] >> 2) * g.ncl[1] + (ic[1] >> 2);
-        key = cl * 16 + 4 * (ic[0] & 3) + (ic[1] & 3);
-    }
-    const int p = (pc[0] * g.npatch[1] + pc[1]) * g.npatch[2] + pc[2];
-    keys[i] = (13u << 27) | (uint32_t)((int64_t)p * g.cpp + key);
+    keys[i] = (13u << 27) | dev::position_key<ND>(g, x);
 }
 
 inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }

@@ -9,7 +9,7 @@ namespace smi {
 
 namespace {
 
-constexpr uint64_t kKeep = 64ull << 20;  // bytes a pool holds between calls
+constexpr uint64_t kKeep = 256ull << 20;  // bytes a pool holds between calls
 
 std::mutex g_lock;
 std::vector<hipMemPool_t> g_pool;  // by device; made at the first use, held until the process ends
