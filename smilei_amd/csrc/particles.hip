@@ -67,6 +67,71 @@ __device__ inline void deposit3_tile(double *sJ, const Geom &g, const int *G0, c
     });
 }
 
+// The 2D J tile: rows of 12 words and four copies 112 words apart, the lane
+// picking its copy: a cluster has 16 cells only, so that four neighbouring
+// lanes of a wavefront share a cell (lane-interleaved storage) and met on the
+// same words.  At one stencil offset the 64 lanes then spread two to a bank
+// pair.
+constexpr int kTile2Row = 12, kTile2Copy = 112, kTile2Copies = 4;
+
+// 2D3V Esirkepov currents (Projector2D2Order.cpp:131-188) of one particle
+// into its copy of the tile, transverse weights and current factors
+// factorised as esirkepov3d_fact; NT = 3: the node is unchanged on both axes
+// (21 adds), NT = 4 otherwise (40).  The walk of all 65 points with a test for
+// zero at each, on one copy of the tile, took 594 us a step for 8.4e6
+// particles, this 490.
+template <int NT>
+__device__ inline void deposit2_tile(double *sJ, const Geom &g, const int *G0, const double *dold, const double *pnn,
+                                     const int *ip, double cw, double crz)
+{
+    constexpr int NA = NT - 1;
+    double S0[2][4], DS[2][4];
+    int w0[2] = {1, 1};
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+        if constexpr (NT == 3) {
+            double s1[3];
+            spline<2>(dold[d], S0[d]);
+            spline<2>(pnn[d] - (double)ip[d], s1);
+#pragma unroll
+            for (int m = 0; m < 3; ++m) DS[d][m] = s1[m] - S0[d][m];
+        } else {
+            esirkepov_window<2>(dold[d], pnn[d], ip[d], S0[d], DS[d], w0[d]);
+        }
+    }
+    constexpr int C = kTile2Copies * kTile2Copy;
+    double *t = sJ + (threadIdx.x & (kTile2Copies - 1)) * kTile2Copy + (ip[0] - G0[0] + w0[0]) * kTile2Row +
+                (ip[1] - G0[1] + w0[1]);
+    const double cr[2] = {cw * g.dxdt[0], cw * g.dxdt[1]};
+    double A[2][NA], M[2][NT];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+        double ps = 0.;
+#pragma unroll
+        for (int r = 0; r < NA; ++r) {
+            ps += DS[d][r];
+            A[d][r] = -cr[d] * ps;
+        }
+#pragma unroll
+        for (int m = 0; m < NT; ++m) M[d][m] = fma(0.5, DS[d][m], S0[d][m]);
+    }
+#pragma unroll
+    for (int r = 0; r < NA; ++r)
+#pragma unroll
+        for (int m = 0; m < NT; ++m) {
+            atomicAdd(&t[(r + 1) * kTile2Row + m], A[0][r] * M[1][m]);
+            atomicAdd(&t[C + m * kTile2Row + r + 1], A[1][r] * M[0][m]);
+        }
+    // Jz: crz (S0y (S0x + S1x / 2) + S1y (S0x / 2 + S1x))
+#pragma unroll
+    for (int m = 0; m < NT; ++m) {
+        const double u = crz * fma(0.5, DS[0][m], 1.5 * S0[0][m]), v = crz * fma(1.5, S0[0][m], DS[0][m]);
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+            atomicAdd(&t[2 * C + m * kTile2Row + q], fma(S0[1][q], u, (S0[1][q] + DS[1][q]) * v));
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Fused particle kernel.
 // ---------------------------------------------------------------------------
@@ -90,18 +155,17 @@ __device__ __attribute__((always_inline)) inline void fp_cluster(const Geom &g, 
     constexpr int JT3 = ND == 3 ? JT * JT * JT : JT * JT;
     // 3D order 2: J rows padded by one word, so that the tile atomics of a
     // wavefront meet fewer LDS bank conflicts (the strides of deposit3_tile)
-    constexpr int JSY = ND == 3 && ORDER == 2 ? JT + 1 : JT, JSX = JT * JSY, JSC = ND == 3 ? JT * JSX : JT3;
+    constexpr int JSY = ND == 3 && ORDER == 2 ? JT + 1 : JT, JSX = JT * JSY,
+                  JSC = ND == 3 ? JT * JSX : kTile2Copies * kTile2Copy;
     __shared__ double sF[6 * GF];
     __shared__ double sJ[DEPOSIT ? 3 * JSC : 1];
     __shared__ int sHist[kMaxMerged][64];  // destination-cell counts of this cluster's own cells
-    // 3D deposit: particles whose node changes on some axis are deposited in
-    // a second pass over this queue (old delta, new position in cells, charge
+    // particles whose node changes on some axis are deposited in a second pass over this queue (old delta, new position in cells, charge
     // weight, old node relative to the cluster), so that the main loop runs
     // the narrow stencil with all lanes.  Order 4: a short queue, so that the
     // workgroup's LDS (field and J tiles of 10^3 and 11^3 points) stays within
     // 80 KB and two workgroups fit a CU.
-    constexpr bool QUEUE = DEPOSIT && ND == 3;
-    constexpr int QCAP = QUEUE ? (ORDER == 4 ? 12 : 96) : 1;
+    constexpr int QCAP = DEPOSIT ? (ORDER == 4 ? 12 : 96) : 1;
     __shared__ double sQ[QCAP][8];
     __shared__ int sQn;
 
@@ -290,50 +354,44 @@ __device__ __attribute__((always_inline)) inline void fp_cluster(const Geom &g, 
         } else {
             // ---- Esirkepov currents into the LDS tile
             const double cw = sp.cw_scale * w;
-            if constexpr (ND == 3) {
-                double pnn[3];
-                int moved = 0;
+            const double crz = ND == 2 ? cw * kThird * u[2] * invgf : 0.;
+            double pnn[3];
+            int moved = 0;
 #pragma unroll
-                for (int d = 0; d < 3; ++d) {
-                    pnn[d] = xn[d] * g.dinv[d];
-                    moved |= (int)round(pnn[d]) - ip[d];
-                }
-                if (moved == 0) deposit3_tile<ORDER, ORDER + 1>(sJ, g, cl.G0, dold, pnn, ip, cw);
-                const uint64_t gm = __ballot(moved != 0);
-                if (gm) {
-                    const int lane = threadIdx.x & 63;
-                    const int leader = __ffsll((unsigned long long)gm) - 1;
-                    int base = 0;
-                    if (lane == leader) base = atomicAdd(&sQn, __popcll(gm));
-                    base = __shfl(base, leader, 64);
-                    if (moved != 0) {
-                        const int pos = base + __popcll(gm & ((1ull << lane) - 1));
-                        if (pos < QCAP) {
+            for (int d = 0; d < ND; ++d) {
+                pnn[d] = xn[d] * g.dinv[d];
+                moved |= (int)round(pnn[d]) - ip[d];
+            }
+            if (moved == 0) {
+                if constexpr (ND == 3) deposit3_tile<ORDER, ORDER + 1>(sJ, g, cl.G0, dold, pnn, ip, cw);
+                else deposit2_tile<3>(sJ, g, cl.G0, dold, pnn, ip, cw, crz);
+            }
+            const uint64_t gm = __ballot(moved != 0);
+            if (gm) {
+                const int lane = threadIdx.x & 63;
+                const int leader = __ffsll((unsigned long long)gm) - 1;
+                int base = 0;
+                if (lane == leader) base = atomicAdd(&sQn, __popcll(gm));
+                base = __shfl(base, leader, 64);
+                if (moved != 0) {
+                    const int pos = base + __popcll(gm & ((1ull << lane) - 1));
+                    if (pos < QCAP) {
+                        int packed = 0;
 #pragma unroll
-                            for (int d = 0; d < 3; ++d) {
-                                sQ[pos][d] = dold[d];
-                                sQ[pos][3 + d] = pnn[d];
-                            }
-                            sQ[pos][6] = cw;
-                            sQ[pos][7] = (double)((ip[0] - cl.G0[0]) | ((ip[1] - cl.G0[1]) << 4) |
-                                                  ((ip[2] - cl.G0[2]) << 8));
-                        } else {
-                            deposit3_tile<ORDER, ORDER + 2>(sJ, g, cl.G0, dold, pnn, ip, cw);
+                        for (int d = 0; d < ND; ++d) {
+                            sQ[pos][d] = dold[d];
+                            sQ[pos][3 + d] = pnn[d];
+                            packed |= (ip[d] - cl.G0[d]) << (4 * d);
                         }
+                        if constexpr (ND == 2) sQ[pos][2] = crz;
+                        sQ[pos][6] = cw;
+                        sQ[pos][7] = (double)packed;
+                    } else if constexpr (ND == 3) {
+                        deposit3_tile<ORDER, ORDER + 2>(sJ, g, cl.G0, dold, pnn, ip, cw);
+                    } else {
+                        deposit2_tile<4>(sJ, g, cl.G0, dold, pnn, ip, cw, crz);
                     }
                 }
-            } else {
-                double S0[3][7], S1[3][7], DS[3][7];
-#pragma unroll
-                for (int d = 0; d < ND; ++d)
-                    esirkepov_shapes<ORDER>(dold[d], xn[d] * g.dinv[d], ip[d], S0[d], S1[d], DS[d]);
-                const double crx = cw * (g.dx[0] / g.dt), cry = cw * (g.dx[1] / g.dt);
-                const double crz = cw * kThird * u[2] * invgf;
-                const int o0 = ip[0] - 2 - (cl.G0[0] - TL::JO);
-                const int o1 = ip[1] - 2 - (cl.G0[1] - TL::JO);
-                esirkepov2d(S0, S1, DS, crx, cry, crz, [&](int c, int a, int b, double v) {
-                    if (v != 0.) atomicAdd(&sJ[c * JT3 + (o0 + a) * JT + (o1 + b)], v);
-                });
             }
         }
     }
@@ -349,7 +407,7 @@ __device__ __attribute__((always_inline)) inline void fp_cluster(const Geom &g, 
             if (S.stay) S.stay[cl.gbase + t % 64] = (uint8_t)(c < (int)kPlaceMax ? c : (int)kPlaceMax);
         }
     }
-    if constexpr (QUEUE) {
+    if constexpr (DEPOSIT) {
         const int nq = sQn < QCAP ? sQn : QCAP;
         for (int t = threadIdx.x; t < nq; t += blockDim.x) {
             const double dold[3] = {sQ[t][0], sQ[t][1], sQ[t][2]};
@@ -357,11 +415,10 @@ __device__ __attribute__((always_inline)) inline void fp_cluster(const Geom &g, 
             const int packed = (int)sQ[t][7];
             const int ip[3] = {cl.G0[0] + (packed & 15), cl.G0[1] + ((packed >> 4) & 15),
                                cl.G0[2] + ((packed >> 8) & 15)};
-            deposit3_tile<ORDER, ORDER + 2>(sJ, g, cl.G0, dold, pnn, ip, sQ[t][6]);
+            if constexpr (ND == 3) deposit3_tile<ORDER, ORDER + 2>(sJ, g, cl.G0, dold, pnn, ip, sQ[t][6]);
+            else deposit2_tile<4>(sJ, g, cl.G0, dold, pnn, ip, sQ[t][6], sQ[t][2]);
         }
         __syncthreads();
-    }
-    if constexpr (DEPOSIT) {
         // one tile position per thread and pass, its grid index computed once
         // for the three components (32-bit: the engine holds fewer than 2^27
         // cells)
@@ -383,7 +440,14 @@ __device__ __attribute__((always_inline)) inline void fp_cluster(const Geom &g, 
             const int idx = (gi * g.N[1] + gj) * g.N[2] + gk;
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                const double v = ND == 3 ? sJ[c * JSC + a * JSX + b * JSY + k] : sJ[c * JT3 + r];
+                double v;
+                if constexpr (ND == 3) {
+                    v = sJ[c * JSC + a * JSX + b * JSY + k];
+                } else {
+                    v = 0.;
+#pragma unroll
+                    for (int q = 0; q < kTile2Copies; ++q) v += sJ[c * JSC + q * kTile2Copy + a * kTile2Row + b];
+                }
                 if (v != 0.) unsafeAtomicAdd((double *)(dstJ[c] + idx), v);
             }
         }

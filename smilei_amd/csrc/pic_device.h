@@ -141,7 +141,7 @@ __device__ inline int32_t cell_key(const Geom &g, const int *pc, const double *x
     int ic[3] = {0, 0, 0};
 #pragma unroll
     for (int d = 0; d < ND; ++d) {
-        int c = (int)floor(x[d] * (1.0 / g.dx[d])) - pc[d] * g.n[d];
+        int c = (int)floor(x[d] * g.dinv[d]) - pc[d] * g.n[d];
         c = c < 0 ? 0 : (c > g.n[d] - 1 ? g.n[d] - 1 : c);
         ic[d] = c;
     }
@@ -166,7 +166,7 @@ __device__ inline uint32_t position_key(const Geom &g, const double *x)
         while (c > 0 && x[d] < (double)c * g.plen[d]) --c;
         while (c < g.npatch[d] - 1 && x[d] >= (double)(c + 1) * g.plen[d]) ++c;
         pc[d] = c;
-        int k = (int)floor(x[d] * (1.0 / g.dx[d])) - c * g.n[d];
+        int k = (int)floor(x[d] * g.dinv[d]) - c * g.n[d];
         ic[d] = k < 0 ? 0 : (k > g.n[d] - 1 ? g.n[d] - 1 : k);
     }
     int key;
