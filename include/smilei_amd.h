@@ -195,7 +195,11 @@ int smi_profile_step(smi_context *ctx, float *ms);
 /* The stream all work of the context is enqueued on (hipStream_t). */
 void *smi_stream(smi_context *ctx);
 /* Launch-shape knobs of the particle kernels, searched by smi_autotune (no
- * effect on results beyond the order of the atomic J summation).
+ * effect on results beyond the order of the atomic J summation).  Until
+ * SMI_TUNE_THREADS, or SMI_TUNE_INTERLEAVE and SMI_TUNE_TILE, are set (or the
+ * autotuner has run), grid launches take the workgroup size, layout and tile
+ * from the geometry and the order; the starting values that smi_get_tuning
+ * reports then are those of the other launches.
  * SMI_TUNE_INTERLEAVE (mixed form and atomic FP64 form): 1 = the sort
  * stores each cluster's particles lane-interleaved (64 columns of
  * consecutive cell-sorted ranks, stored row by row), so that the 64 lanes of

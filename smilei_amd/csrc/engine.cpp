@@ -104,6 +104,7 @@ struct smi_context {
     int tile = 1;                  // J-tile shape of the mixed kernel: rows padded by one word (tuning)
     int tile_x = 1;                // patch-tile extent of the mixed kernel: clusters along x per workgroup (tuning)
     int node_acc = 0;              // mixed kernel: stayers' tile words summed node by node (tuning)
+    bool interleave_set = false, threads_set = false, tile_set = false;  // chosen by the caller or the autotuner
     int persistent_blocks = 0;     // its grid, from the occupancy of the current knobs
     int *d_work = nullptr;         // work list (one int per cluster) + head/count (2 ints)
     hipGraphExec_t graph[2] = {nullptr, nullptr};
@@ -129,12 +130,49 @@ void check_ctx(const smi_context *c)
     if (!c) throw Error(SMI_ERR_INVALID, "null context");
 }
 
+// Launch shape of a grid launch where nobody has chosen one (the persistent,
+// node-accumulated and two-cluster forms keep the knobs' values).  One step's particle kernel, microseconds:
+//  * Order-4 mixed form: pair-interleaved layout and unpadded J rows, whose
+//    pre-reduction halves the tile atomics that bound it: 4.2e6 particles 779
+//    against 929 lane-interleaved and padded (920 unpadded; pairs, padded 956).
+//  * Up to one cluster per CU (256) the chip is not full and 512 threads
+//    shorten each cluster's work: 16^3 cells of 2 x 8 particles, mixed order 2
+//    32 against 39 at 256 threads, FP64 48 against 58, mixed order 4 83 against
+//    98; the mixed order-2 kernel, whose workgroups are the smallest, gains up
+//    to two per CU (32^3 cells 45 against 50; FP64 90 against 80, order 4 158
+//    against 146; at three per CU 68 against 61).
+//  * 2D clusters hold 16 cells: 128 threads, unless they are crowded (256^2
+//    cells of 2 x 4 particles 58 against 84 at 256 threads, 2 x 16 116 against
+//    125, 2 x 64 405 against 384; 1024^2 cells of 2 x 16 1,575 against 1,916).
+bool pair_default(const smi_context *c)
+{
+    return c->mixed && c->g.order == 4 && !c->persistent && !c->interleave_set && !c->tile_set;
+}
+
+int launch_threads(const smi_context *c)
+{
+    if (c->threads_set || c->persistent || c->node_acc || c->tile_x != 1) return c->threads;
+    const Geom &g = c->g;
+    const int64_t clusters = (int64_t)g.npatches * g.clpp, cus = 256;
+    const int64_t few = c->mixed && g.order == 2 ? 2 * cus : cus;
+    if (clusters <= few) return std::min(512, particle_max_threads(g, c->mixed));
+    if (g.nd == 2) {
+        int64_t n = 0;
+        for (int id : c->moving) n += c->sp[id].n;
+        return n <= 1024 * clusters ? 128 : 256;
+    }
+    return c->threads;
+}
+
+int launch_tile(const smi_context *c) { return pair_default(c) ? 0 : c->tile; }
+
 // Cluster layout the tile-deposit kernels (mixed form, atomic FP64 form)
 // read: the tuning's (lane-interleaved by default); the deterministic
 // deposit walks the cells in order and keeps cell-major order (0).
 int want_interleaved(const smi_context *c)
 {
-    return c->p.deposit != SMI_DEPOSIT_DETERMINISTIC ? c->interleave : 0;
+    if (c->p.deposit == SMI_DEPOSIT_DETERMINISTIC) return 0;
+    return pair_default(c) ? 2 : c->interleave;
 }
 
 // The particle kernel records each input particle's cell-major position
@@ -248,8 +286,9 @@ void enqueue_particles(smi_context *c, int a)
             const bool paired = want_interleaved(c) == 2;
             // the node-accumulated deposit where the launch allows it, else
             // the per-particle one
-            const bool na = c->node_acc && mixed_node_acc_ok(g, c->threads, tx, paired, c->persistent != 0);
-            launch_particles_mixed(g, c->d_mix + a * ns + g0, n, cr_max, GF, J, c->err, c->threads, c->xcd != 0, c->tile,
+            const int threads = launch_threads(c);
+            const bool na = c->node_acc && mixed_node_acc_ok(g, threads, tx, paired, c->persistent != 0);
+            launch_particles_mixed(g, c->d_mix + a * ns + g0, n, cr_max, GF, J, c->err, threads, c->xcd != 0, launch_tile(c),
                                    tx, paired, na, c->persistent ? c->persistent_blocks : 0, c->d_work,
                                    c->d_work + g.npatches * g.clpp, c->st);
         }
@@ -257,7 +296,7 @@ void enqueue_particles(smi_context *c, int a)
         const int ns = (int)c->moving.size();
         for (int g0 = 0; g0 < ns; g0 += kMaxMerged)
             launch_particles(g, c->d_fp + a * ns + g0, std::min(kMaxMerged, ns - g0), GF, J, !det, c->err,
-                             c->threads, c->xcd != 0, c->persistent ? c->persistent_blocks : 0, c->d_work,
+                             launch_threads(c), c->xcd != 0, c->persistent ? c->persistent_blocks : 0, c->d_work,
                              c->d_work + g.npatches * g.clpp, c->st);
     }
 }
@@ -1215,6 +1254,7 @@ int smi_set_tuning(smi_context *c, int key, int value)
         if (value == 2 && !c->mixed)
             throw Error(SMI_ERR_INVALID, "SMI_TUNE_INTERLEAVE = 2 (pair-interleaved) is a mixed-form layout");
         c->interleave = value;
+        c->interleave_set = true;
     } else if (key == SMI_TUNE_THREADS) {
         if (value != 64 && value != 128 && value != 256 && value != 512)
             throw Error(SMI_ERR_INVALID, "SMI_TUNE_THREADS must be 64, 128, 256 or 512");
@@ -1222,6 +1262,7 @@ int smi_set_tuning(smi_context *c, int key, int value)
             throw Error(SMI_ERR_INVALID, "SMI_TUNE_THREADS above the particle kernel's limit (256 for the 3D "
                                          "order-4 FP64 kernel)");
         c->threads = value;
+        c->threads_set = true;
     } else if (key == SMI_TUNE_CELL_ORDER) {
         c->cell_order = value != 0;
     } else if (key == SMI_TUNE_XCD) {
@@ -1231,6 +1272,7 @@ int smi_set_tuning(smi_context *c, int key, int value)
     } else if (key == SMI_TUNE_TILE) {
         if (value != 0 && value != 1) throw Error(SMI_ERR_INVALID, "SMI_TUNE_TILE must be 0 or 1");
         c->tile = value;
+        c->tile_set = true;
     } else if (key == SMI_TUNE_TILE_X) {
         if (value != 1 && value != 2) throw Error(SMI_ERR_INVALID, "SMI_TUNE_TILE_X must be 1 or 2");
         if (value == 2 && !(c->mixed && mixed_tile_x_ok(c->g, 2, false)))
@@ -1301,8 +1343,9 @@ int smi_autotune(smi_context *c, int reps, float *best_ms)
     // node-accumulated deposit: mixed form, order 2
     const int nna = c->mixed && c->g.order == 2 ? 2 : 1;
     float best = 3.4e38f;
+    c->interleave_set = c->threads_set = c->tile_set = true;
     for (int m = 0; m < nmap; ++m) {
-    if (!det && c->interleave != maps[m]) {
+    if (!det) {
         c->interleave = maps[m];
         apply_layout(c);
     }
