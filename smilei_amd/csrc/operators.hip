@@ -25,9 +25,10 @@ struct Dbl3 {
 
 // Interpolator3D{2,4}Order::fieldsWrapper, one thread per particle.
 // (launched with 256 threads: the bound leaves the compiler 256 registers
-// instead of the 128 of a 1024-thread default, so nothing spills)
-template <int ORDER>
-__global__ void __launch_bounds__(256, 2) k_interp3d(const double *Ex, const double *Ey, const double *Ez, const double *Bx, const double *By,
+// instead of the 128 of a 1024-thread default; the six gathers are kept apart,
+// so that their loads in flight fit in them)
+template <int ORDER, class O>
+__global__ void __launch_bounds__(256, ORDER == 4 ? 3 : 4) k_interp3d(const double *Ex, const double *Ey, const double *Ez, const double *Bx, const double *By,
                            const double *Bz, Ints3 np, Ints3 dom, Dbl3 dinv, int64_t n, const double *x,
                            const double *y, const double *z, double *Ep, double *Bp, int32_t *iold, double *dold)
 {
@@ -55,12 +56,12 @@ __global__ void __launch_bounds__(256, 2) k_interp3d(const double *Ex, const dou
         return;
     }
     const int ny = np.v[1], nz = np.v[2];
-    Ep[i] = gather3s<H>(cd[0], cp[1], cp[2], Ex, id[0], ip[1], ip[2], ny, nz);
-    Ep[n + i] = gather3s<H>(cp[0], cd[1], cp[2], Ey, ip[0], id[1], ip[2], ny + 1, nz);
-    Ep[2 * n + i] = gather3s<H>(cp[0], cp[1], cd[2], Ez, ip[0], ip[1], id[2], ny, nz + 1);
-    Bp[i] = gather3s<H>(cp[0], cd[1], cd[2], Bx, ip[0], id[1], id[2], ny + 1, nz + 1);
-    Bp[n + i] = gather3s<H>(cd[0], cp[1], cd[2], By, id[0], ip[1], id[2], ny, nz + 1);
-    Bp[2 * n + i] = gather3s<H>(cd[0], cd[1], cp[2], Bz, id[0], id[1], ip[2], ny + 1, nz);
+    Ep[i] = gather3s<H, O>(cd[0], cp[1], cp[2], Ex, id[0], ip[1], ip[2], ny, nz);
+    Bp[n + i] = gather3s<H, O>(cd[0], cp[1], cd[2], By, id[0], ip[1], id[2], ny, nz + 1);
+    Ep[n + i] = gather3s<H, O>(cp[0], cd[1], cp[2], Ey, ip[0], id[1], ip[2], ny + 1, nz);
+    Bp[i] = gather3s<H, O>(cp[0], cd[1], cd[2], Bx, ip[0], id[1], id[2], ny + 1, nz + 1);
+    Ep[2 * n + i] = gather3s<H, O>(cp[0], cp[1], cd[2], Ez, ip[0], ip[1], id[2], ny, nz + 1);
+    Bp[2 * n + i] = gather3s<H, O>(cd[0], cd[1], cp[2], Bz, id[0], id[1], ip[2], ny + 1, nz);
     for (int d = 0; d < 3; ++d) {
         iold[d * n + i] = ip[d];
         dold[d * n + i] = dp[d];
@@ -592,12 +593,19 @@ int smi_interpolate_3d(int order, const double *Ex, const double *Ey, const doub
     Ints3 NP{{np[0], np[1], np[2]}}, D{{dom_begin[0], dom_begin[1], dom_begin[2]}};
     Dbl3 di{{1.0 / cell_length[0], 1.0 / cell_length[1], 1.0 / cell_length[2]}};
     hipStream_t st = (hipStream_t)stream;
-    if (order == 2)
-        hipLaunchKernelGGL(k_interp3d<2>, dim3(nblk(n, 256)), dim3(256), 0, st, Ex, Ey, Ez, Bxm, Bym, Bzm, NP, D, di,
-                           n, x, y, z, Epart, Bpart, iold, deltaold);
-    else
-        hipLaunchKernelGGL(k_interp3d<4>, dim3(nblk(n, 256)), dim3(256), 0, st, Ex, Ey, Ez, Bxm, Bym, Bzm, NP, D, di,
-                           n, x, y, z, Epart, Bpart, iold, deltaold);
+    const dim3 grid(nblk(n, 256)), block(256);
+    const bool small = (int64_t)(np[0] + 1) * (np[1] + 1) * (np[2] + 1) < (1ll << 29);
+#define SMI_INTERP(O, T)                                                                                             \
+    hipLaunchKernelGGL((k_interp3d<O, T>), grid, block, 0, st, Ex, Ey, Ez, Bxm, Bym, Bzm, NP, D, di, n, x, y, z, Epart, \
+                       Bpart, iold, deltaold)
+    if (order == 2) {
+        if (small) SMI_INTERP(2, uint32_t);
+        else SMI_INTERP(2, uint64_t);
+    } else {
+        if (small) SMI_INTERP(4, uint32_t);
+        else SMI_INTERP(4, uint64_t);
+    }
+#undef SMI_INTERP
     OP_CHECK();
     return SMI_OK;
 }

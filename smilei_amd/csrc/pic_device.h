@@ -235,18 +235,25 @@ __device__ inline double gather2(const double *cx, const double *cy, const doubl
 }
 
 // Same gathers on a strided array (the reference's per-patch Field3D/2D).
-template <int H>
+// O: unsigned 32-bit byte offsets from the array's scalar base where the array
+// is below 4 GiB, one add per row; 64-bit ones otherwise.
+template <int H, class O>
 __device__ inline double gather3s(const double *cx, const double *cy, const double *cz, const double *f, int i,
                                   int j, int k, int ny, int nz)
 {
+    const O sy = (O)nz * 8, sx = (O)ny * sy;
+    const O at = ((O)(i - H) * ny + (j - H)) * sy + (O)(k - H) * 8;
     double r = 0.;
 #pragma unroll
-    for (int a = -H; a <= H; ++a)
+    for (int a = -H; a <= H; ++a) {
+        if constexpr (H == 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int b = -H; b <= H; ++b)
+        for (int b = -H; b <= H; ++b) {
+            const double *row = (const double *)((const char *)f + (O)(at + (O)(a + H) * sx + (O)(b + H) * sy));
 #pragma unroll
-            for (int c = -H; c <= H; ++c)
-                r += cx[a + H] * cy[b + H] * cz[c + H] * f[((int64_t)(i + a) * ny + (j + b)) * nz + (k + c)];
+            for (int c = -H; c <= H; ++c) r += cx[a + H] * cy[b + H] * cz[c + H] * row[c + H];
+        }
+    }
     return r;
 }
 
