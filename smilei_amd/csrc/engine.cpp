@@ -21,6 +21,7 @@
 
 #include "../../include/smilei_amd.h"
 #include "kernels.h"
+#include "readback.h"
 
 using namespace smi;
 
@@ -89,7 +90,7 @@ struct smi_context {
     int d_det_n = 0;
     MixSpecies *d_mix = nullptr;   // mixed-form particle-launch descriptors [2][species]
     FpSpecies *d_fp = nullptr;     // FP64-form particle-launch descriptors [2][species]
-    double *partials = nullptr;    // reduction scratch
+    double *partials = nullptr;    // reduction scratch: kReduceBlocks for the fields and for each species
     double *rho = nullptr;         // diagnostics scratch (ncells)
     int *err = nullptr;            // device flag raised by kernels on corrupt particles
     int cur = 0;                   // particle buffer holding the current state
@@ -109,6 +110,7 @@ struct smi_context {
     int *d_work = nullptr;         // work list (one int per cluster) + head/count (2 ints)
     hipGraphExec_t graph[2] = {nullptr, nullptr};
     hipEvent_t ev[6] = {};
+    Readback back;                 // fields, density and reductions to the host
 
     FieldSet fields() const
     {
@@ -539,6 +541,7 @@ int smi_create(const smi_params *p, smi_context **out)
             launch_fill(c->F[f], ncells, 0.0, c->st);
         }
         c->partials = dalloc<double>(kReduceBlocks);
+        c->back.init(ncells * sizeof(double));
         c->rho = dalloc<double>(ncells);
         c->err = dalloc<int>(1);
         launch_fill_i32(c->err, 1, 0, c->st);
@@ -586,6 +589,7 @@ int smi_destroy(smi_context *c)
     (void)hipFree(c->err);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);
+    c->back.release();
     if (c->st) (void)hipStreamDestroy(c->st);
     delete c;
     return SMI_OK;
@@ -636,6 +640,10 @@ int smi_add_species(smi_context *c, const char *name, double mass, double charge
     s.km.cwd = s.k.cw_scale;
     for (int d = 0; d < 3; ++d) s.km.dxdt[d] = (float)(c->g.dx[d] / c->g.dt);
     set_quantum(c->g, s, 1.0);
+    double *partials = dalloc<double>((2 + (int64_t)c->sp.size()) * kReduceBlocks);
+    SMI_HIP(hipStreamSynchronize(c->st));
+    (void)hipFree(c->partials);
+    c->partials = partials;
     c->sp.push_back(s);
     c->moving = moving_now(c);
     // deterministic-deposit descriptors for both ping-pong parities
@@ -1141,8 +1149,7 @@ int smi_get_field(smi_context *c, int f, double *gl)
     check_ctx(c);
     if (f < 0 || f >= SMI_NFIELDS || !gl) throw Error(SMI_ERR_INVALID, "bad field id");
     SMI_HIP(hipSetDevice(c->p.device));
-    SMI_HIP(hipStreamSynchronize(c->st));
-    SMI_HIP(hipMemcpy(gl, c->F[f], c->g.ncells * sizeof(double), hipMemcpyDeviceToHost));
+    c->back.copy(gl, c->F[f], c->g.ncells * sizeof(double), c->st);
     return SMI_OK;
     SMI_CATCH
 }
@@ -1453,26 +1460,25 @@ int smi_energies(smi_context *c, double *out)
     SMI_TRY
     check_ctx(c);
     SMI_HIP(hipSetDevice(c->p.device));
-    std::vector<double> h(kReduceBlocks);
+    // every reduction's partial sums side by side, one copy to the host
+    const int64_t nred = 1 + (int64_t)c->sp.size();
     const int fid[6] = {SMI_EX, SMI_EY, SMI_EZ, SMI_BXM, SMI_BYM, SMI_BZM};
     const double *fl[6] = {c->F[SMI_EX], c->F[SMI_EY], c->F[SMI_EZ], c->F[SMI_BXM], c->F[SMI_BYM], c->F[SMI_BZM]};
     launch_sumsq(c->g, fl, fid, 6, c->partials, kReduceBlocks, c->st);
-    SMI_HIP(hipMemcpyAsync(h.data(), c->partials, kReduceBlocks * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    SMI_HIP(hipStreamSynchronize(c->st));
-    double s = 0;
-    for (double v : h) s += v;
-    double cell_volume = 1.0;
-    for (int d = 0; d < c->g.nd; ++d) cell_volume *= c->g.dx[d];
-    out[0] = 0.5 * cell_volume * s;
     for (size_t k = 0; k < c->sp.size(); ++k) {
         SpeciesState &S = c->sp[k];
-        if (c->mixed) launch_ukin_mixed(S.mview(c->cur), S.sb.perm, S.n, c->partials, kReduceBlocks, c->st);
-        else launch_ukin(S.view(c->cur), S.sb.perm, S.n, c->partials, kReduceBlocks, c->st);
-        SMI_HIP(hipMemcpyAsync(h.data(), c->partials, kReduceBlocks * sizeof(double), hipMemcpyDeviceToHost, c->st));
-        SMI_HIP(hipStreamSynchronize(c->st));
-        double e = 0;
-        for (double v : h) e += v;
-        out[1 + k] = e * S.mass;
+        double *part = c->partials + (1 + k) * kReduceBlocks;
+        if (c->mixed) launch_ukin_mixed(S.mview(c->cur), S.sb.perm, S.n, part, kReduceBlocks, c->st);
+        else launch_ukin(S.view(c->cur), S.sb.perm, S.n, part, kReduceBlocks, c->st);
+    }
+    std::vector<double> h(nred * kReduceBlocks);
+    c->back.copy(h.data(), c->partials, h.size() * sizeof(double), c->st);
+    double cell_volume = 1.0;
+    for (int d = 0; d < c->g.nd; ++d) cell_volume *= c->g.dx[d];
+    for (int64_t q = 0; q < nred; ++q) {
+        double s = 0;
+        for (int i = 0; i < kReduceBlocks; ++i) s += h[q * kReduceBlocks + i];
+        out[q] = q == 0 ? 0.5 * cell_volume * s : s * c->sp[q - 1].mass;
     }
     return SMI_OK;
     SMI_CATCH
@@ -1496,8 +1502,7 @@ int smi_rho(smi_context *c, double *gl)
     check_ctx(c);
     SMI_HIP(hipSetDevice(c->p.device));
     compute_rho(c);
-    SMI_HIP(hipMemcpyAsync(gl, c->rho, c->g.ncells * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    SMI_HIP(hipStreamSynchronize(c->st));
+    c->back.copy(gl, c->rho, c->g.ncells * sizeof(double), c->st);
     return SMI_OK;
     SMI_CATCH
 }
@@ -1509,8 +1514,7 @@ int smi_gauss(smi_context *c, double *gl)
     SMI_HIP(hipSetDevice(c->p.device));
     compute_rho(c);
     launch_gauss(c->g, c->fields(), c->rho, c->st);
-    SMI_HIP(hipMemcpyAsync(gl, c->rho, c->g.ncells * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    SMI_HIP(hipStreamSynchronize(c->st));
+    c->back.copy(gl, c->rho, c->g.ncells * sizeof(double), c->st);
     return SMI_OK;
     SMI_CATCH
 }
