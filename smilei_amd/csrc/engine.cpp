@@ -1491,7 +1491,7 @@ static void compute_rho(smi_context *c)
         if (c->mixed) launch_rho_mixed(c->g, S.km, S.mview(c->cur), S.keys[c->cur], S.sb.perm, S.sb.cell_off, S.n, c->rho,
                                       c->st);
         else if (c->p.deposit == SMI_DEPOSIT_DETERMINISTIC)
-            launch_rho_gather(c->g, S.k, S.view(c->cur), S.sb.perm, S.sb.cell_off, S.lay, c->rho, c->st);
+            launch_rho_gather(c->g, S.k, S.view(c->cur), S.sb.perm, S.sb.cell_off, c->rho, c->st);
         else launch_rho(c->g, S.k, S.view(c->cur), S.sb.perm, S.sb.cell_off, S.n, c->rho, c->st);
     }
 }

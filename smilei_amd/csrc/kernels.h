@@ -307,10 +307,10 @@ void launch_wsum(const double *w, const float *wf, int64_t n, double *partials, 
 // cell_off / perm as the sort left them (any cluster layout).
 void launch_rho(const Geom &g, const SpeciesK &sp, const PartPtrs &A, const int32_t *perm, const int32_t *cell_off,
                 int64_t n, double *rho, hipStream_t st);
-// Same density added in a fixed order (one thread per node gathering from
-// the sorted cells; cell_off / perm / lay as the sort left them).
+// Same density added in a fixed order (each node gathers from the sorted
+// cells; cell_off / perm as the sort left them, cell-major).
 void launch_rho_gather(const Geom &g, const SpeciesK &sp, const PartPtrs &A, const int32_t *perm,
-                       const int32_t *cell_off, int lay, double *rho, hipStream_t st);
+                       const int32_t *cell_off, double *rho, hipStream_t st);
 void launch_gauss(const Geom &g, const FieldSet &f, double *rho_to_residual, hipStream_t st);
 
 }  // namespace smi

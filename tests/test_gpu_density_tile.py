@@ -81,3 +81,48 @@ def test_density_tile(form, order, shape, patch, layout):
     got = sim.rho().reshape(shape[:nd])
     tol = 1e-6 if form == "mixed" else 2e-13
     assert np.abs(got - want).max() <= tol * np.abs(want).max()
+
+
+@pytest.mark.parametrize("shape,patch", [((8, 8, 12), (8, 8, 12)), ((16, 8, 8), (8, 8, 8)), ((20, 12), (20, 12)),
+                                         ((8, 16), (8, 8))])
+def test_deterministic_density_is_the_ordered_sum(shape, patch):
+    """The fixed-order density, bit for bit: per node, the cells that reach it
+    in x, y, z order, their particles in sorted order, products ((cw Sx) Sy) Sz."""
+    nd = len(shape)
+    dx = (0.2, 0.25, 0.3)[:nd]
+    sim = sa.Simulation("%dDcartesian" % nd, 2, shape, patch, dx, cfl_dt(dx), deposit=sa.DEPOSIT_DETERMINISTIC)
+    pos, w = positions(shape + (1,) * (3 - nd), dx, 5)
+    pos, w = [v[:400] for v in pos], w[:400]
+    sid = sim.add_species("s", 1.0, -2.0, len(w))
+    zero = np.zeros(len(w))
+    sim.set_particles(sid, pos[0], pos[1], pos[2] if nd == 3 else zero, zero, zero, zero, w)
+    p = sim.get_particles(sid)
+    x = [p[k] for k in "xyz"[:nd]]
+    dinv = [1.0 / v for v in dx]
+    node = [np.floor(x[d] * dinv[d] + 0.5).astype(int) for d in range(nd)]
+    cell = [np.minimum(np.floor(x[d] * dinv[d]).astype(int), shape[d] - 1) for d in range(nd)]
+    S = []
+    for d in range(nd):
+        e = x[d] * dinv[d] - node[d]
+        S.append([0.5 * (e * e - e + 0.25), 0.75 - e * e, 0.5 * (e * e + e + 0.25)])
+    vol = 1.0
+    for v in dx:
+        vol *= v
+    cw = (1.0 / vol * -2.0) * p["w"]
+    by_cell = {}
+    for i, c in enumerate(zip(*cell)):
+        by_cell.setdefault(c, []).append(i)
+    want = np.zeros(shape)
+    for n in np.ndindex(*shape):
+        acc = 0.0
+        for off in np.ndindex(*([4] * nd)):
+            cu = [n[d] - 2 + off[d] for d in range(nd)]
+            for i in by_cell.get(tuple(cu[d] % shape[d] for d in range(nd)), ()):
+                o = [n[d] - (node[d][i] + cu[d] - cu[d] % shape[d] - 1) for d in range(nd)]
+                if all(0 <= v < 3 for v in o):
+                    t = cw[i]
+                    for d in range(nd):
+                        t = t * S[d][o[d]][i]
+                    acc += t
+        want[n] = acc
+    assert np.array_equal(sim.rho().reshape(shape), want)
