@@ -267,19 +267,25 @@ struct MixTile {
     // x extents of a tile of TX clusters along x
     static constexpr int GTX = 4 * TX + 2 * H + 2, JTX = 4 * TX + 2 * H + 2;
     static constexpr int GSY = GT, GSX = ORDER == 2 ? 76 : GT * GT, GF = GTX * GSX;
-    // padded shape: rows of JT + 2 words and x-planes of 104 (order 2) or
-    // 136 (order 4) words, the strides for which the 64 nodes of a cluster,
-    // at one common stencil offset (the lanes of one atomic instruction),
-    // spread evenly over the LDS banks (each 8-byte word address mod 32 hit
-    // by two lanes, the fewest possible for 64 lanes; with unpadded x-planes
-    // of JT * JT words, three or four).  Measured on the beam-plasma: 8 rows
-    // of 10 words in x-planes of 104 (order 2) 49.0 ms, x-planes of 88 49.2,
-    // unpadded rows of 8 in planes of 66 (also two lanes per bank pair at one
-    // offset) 54.2, the earlier 9 rows of 10 in planes of 104 50.2.
-    // (order 4, unpadded rows: x-planes of 104 words, not 10 x 10 = 100,
-    // for the same spread: 13.45 against 13.77 ms on the thermal plasma)
-    static constexpr int JSY = JT + 2 * JPAD, JSX = JPAD ? (ORDER == 2 ? 104 : 136) : (ORDER == 4 ? 104 : JT * JSY),
-                         JSC = JTX * JSX;
+    // strides for which the 64 nodes of a cluster, at one common stencil
+    // offset (the lanes of one atomic instruction), spread over the LDS banks
+    // (32 banks of one 8-byte word) as evenly as 64 lanes can: two lanes a
+    // bank over the whole wavefront and also over each half of it.
+    // Order 2, padded: rows of 12 words in x-planes of 112; unpadded: rows of
+    // 8 in planes of 68.  Order 4, padded: rows of 12 in planes of 144.
+    // (Order 4, unpadded: planes of 104 words, two lanes a bank over the
+    // wavefront but four over its halves; the better 144 would cost a third
+    // of the workgroups.)  Measured on a thermal plasma of 2 x 3.4e7
+    // particles (particle kernel, default layout / pair layout; both tiles):
+    //   order 2 padded   104 x 10  3.14 / 3.16 ms   112 x 12  3.08 / 3.10
+    //                     84 x 8   3.36 / 3.13
+    //   order 2 unpadded  64 x 8   3.44 / 3.11      68 x 8   3.36 / 3.09
+    //                     84 x 8   3.36 / 3.15
+    //   order 4 padded   136 x 12 14.05 / 14.06    144 x 12 13.86 / 14.03
+    //   field x-planes of 76 and 68 words 3.08, 66, 70, 74 and 82 3.13,
+    //   72 and 80 3.33
+    static constexpr int JSY = JT + (ORDER == 2 ? 4 : 2) * JPAD;
+    static constexpr int JSX = ORDER == 2 ? (JPAD ? 112 : 68) : (JPAD ? 144 : 104), JSC = JTX * JSX;
     // node accumulation (NACC): per-node staging of the stayers of one
     // 256-particle round, KST entries of 32 bytes per node, and two sets of
     // per-node counters
