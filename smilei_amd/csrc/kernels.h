@@ -101,19 +101,23 @@ int64_t patch_j_size(const Geom &g);  // doubles per patch (Jx+Jy+Jz)
 // particles about n/64 ranks apart, i.e. in different cells: their LDS
 // stencil accesses spread over the tile instead of piling onto the same
 // addresses.  cluster_rank is the inverse map.
+//
+// p / q for 0 <= p, 0 < q.  On the device below 2^21 by the reciprocal:
+// (p + 1/2) / q lies 1/2q or more from an integer, its computed value
+// (p + 1/2) / q * 2e-7 at most from it.
+__host__ __device__ inline int small_div(int p, int q)
+{
+#ifdef __HIP_DEVICE_COMPILE__
+    if (p < (1 << 21)) return (int)(((float)p + 0.5f) * __builtin_amdgcn_rcpf((float)q));
+#endif
+    return p / q;
+}
 __host__ __device__ inline int cluster_slot(int p, int n)
 {
     const int q = (n + 63) >> 6, full = n - 64 * (q - 1);
-    int col, row;
-    if (p < full * q) {
-        col = p / q;
-        row = p - col * q;
-    } else {
-        const int r = p - full * q;
-        const int k = r / (q - 1);
-        col = full + k;
-        row = r - k * (q - 1);
-    }
+    const bool wide = p < full * q;
+    const int d = wide ? q : q - 1, r = wide ? p : p - full * q;
+    const int k = small_div(r, d), row = r - k * d, col = wide ? k : full + k;
     return row * 64 + col;
 }
 __host__ __device__ inline int cluster_rank(int m, int n)
@@ -135,16 +139,9 @@ __host__ __device__ inline int cluster_slot_pair(int p, int n)
     if (p >= 2 * m) return p;
     const int j = p >> 1;
     const int q = (m + 31) >> 5, full = m - 32 * (q - 1);
-    int col, row;
-    if (j < full * q) {
-        col = j / q;
-        row = j - col * q;
-    } else {
-        const int r = j - full * q;
-        const int k = r / (q - 1);
-        col = full + k;
-        row = r - k * (q - 1);
-    }
+    const bool wide = j < full * q;
+    const int d = wide ? q : q - 1, r = wide ? j : j - full * q;
+    const int k = small_div(r, d), row = r - k * d, col = wide ? k : full + k;
     return row * 64 + 2 * col + (p & 1);
 }
 __host__ __device__ inline int cluster_rank_pair(int m, int n)
@@ -174,7 +171,7 @@ struct SortBufs {
     int32_t *perm;     // cap
     int32_t *tmp;      // cap (cell-major order before the interleaved layout)
     int32_t *rank;     // cap (tie-break of the canonical order of the particles that left their cluster)
-    int32_t *big;      // cap / (kFixRegs + 1) + 1, or null: cells too full for the register ranking
+    int32_t *big;      // cap / 17 + 1, or null: cells of more than 256 particles, which a workgroup sorts
     int32_t *nbig;     // 2 (count, queue head of `big`)
     int32_t *bsum;     // scan scratch
     int64_t nbsum;

@@ -303,25 +303,29 @@ __global__ void __launch_bounds__(kScatThreads) k_scatter(SortSet set, int cpc, 
 }
 
 // Canonical order inside a cell: by direction of motion, then source slot.
-// One thread per cell, then one wavefront per crowded cell.  Buckets of up to
-// kFixRegs particles are ranked in registers (all loads issued together, rank
-// = number of smaller (direction, slot) pairs; the pairs are distinct because
-// slots are).  Each wavefront then runs those of its 64 cells that hold up to
-// kFixMid particles, two at a time where each fits in half of its lanes: a
-// lane's rank is counted against the keys of the cell's other lanes, read as
-// scalars.  2D plasma, 2.6e5 cells of 16 particles per species: 104 us per
-// species in two launches with one cell per wavefront at a time, 118 us
-// here for both.  Larger ones go to the work list `big` (count in
-// nbig[0]) for k_bucket_fix_big, or, without a list, to an insertion sort in
-// memory.  The stores of a cell follow the loads of all its places, so the
-// in-place case (dst == src) is safe.
+// A wavefront takes 64 cells, whose particles are one run of places, and works
+// on as many whole cells at a time as fit into kFixBatch places: one lane per
+// place, kFixPer places per lane in flight.  The keys are staged in LDS, and a
+// lane's rank is the number of smaller (direction, slot) pairs of its cell; the
+// pairs are distinct because slots are.  What bounds it is the chain place ->
+// slot -> key of loads from memory, hence the places in flight, eight
+// wavefronts per SIMD (64 registers, one of them spilled; at seven 72 against
+// 54 us) and the 18 KB of LDS.  Cells of more than kFixMid particles go to
+// the work list `big` (count in nbig[0]) for k_bucket_fix_big, or, without a
+// list, to an insertion sort in memory.  The stores of a batch follow the loads
+// of all its places, so the in-place case (dst == src) is safe.
+// 2D plasma, 2 x 2.6e5 cells of 16 particles: 54 us; 118 us with a thread per
+// cell of up to 16 particles and half a wavefront per cell of up to 32.
+// 3D, 2.6e5 cells of 8: 69 -> 29 us; 2 x 4.2e6 cells of 8: 453 -> 378 us.
 // The cell-major input is src; cpc == 0: sorted in place (dst == src);
 // cpc > 0: every particle is written to its lane-interleaved slot of the
 // cluster in dst.  The tie-break value of source slot v is tie[v] when tie
 // is given, else v.
-constexpr int kFixRegs = 16;
 constexpr int kFixMid = 256;
-constexpr int kFixPer = kFixMid / 64;
+constexpr int kFixPer = 8;
+constexpr int kFixBatch = 64 * kFixPer;  // at least kFixMid: a batch holds one cell at least
+constexpr int kFixAhead = 4;             // keys read per step of the ranking
+static_assert(kFixBatch >= kFixMid, "a batch holds whole cells");
 
 // Where the tie-breaks come from: tie[v] (the cell-major position of slot
 // v in the previous sorted order, recorded by the particle kernel), or v
@@ -390,150 +394,128 @@ __device__ inline int wave_append(bool want, int32_t *counter)
     return base + __popcll(m & ((1ull << lane) - 1));
 }
 
-// Key of lane j (the same j for all lanes).
-__device__ inline uint64_t lane_key(uint64_t k, int j)
+// Orders a wavefront's accesses to LDS that only it uses.
+__device__ inline void lds_order()
 {
-    const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)k, j), hi = __builtin_amdgcn_readlane((uint32_t)(k >> 32), j);
-    return ((uint64_t)hi << 32) | lo;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
-__global__ void __launch_bounds__(256) k_bucket_fix(SortSet set, int64_t ncells, int cpc, int lay, TieGeom G)
+// Cells per wavefront for so many cells of all species: 64 where that still
+// gives the chip the 8,192 wavefronts it holds, else 32 or 16.  Measured for
+// 64 / 32 / 16 / 8 cells: 5.2e5 cells 63 / 65 / 67 / 78 us, 2.6e5 cells 42 / 32 /
+// 33 / 38 us, 6.6e4 cells 22 / 14 / 10 / 11 us.
+constexpr int64_t kFixWaves = 8192;
+
+inline int fix_cells(int64_t cells)
+{
+    return cells >= 64 * kFixWaves ? 64 : cells >= 32 * kFixWaves ? 32 : 16;
+}
+
+__global__ void __launch_bounds__(256, 8) k_bucket_fix(SortSet set, int64_t ncells, int wcells, int cpc, int lay, TieGeom G)
 {
     const SortOne &S = set.s[blockIdx.y];
     const uint32_t *__restrict__ keys = S.keys;
     const int32_t *__restrict__ cell_off = S.cell_off;
     int32_t *src = S.first, *dst = S.perm;
     const TieSrc T(S, G);
+    __shared__ uint64_t sKey[4][kFixBatch + kFixAhead];
+    __shared__ __align__(8) uint8_t sHead[4][kFixBatch];
+    uint64_t *const sk = sKey[threadIdx.x >> 6];
+    uint8_t *const sh = sHead[threadIdx.x >> 6];  // 1 + the lane whose cell begins at a place, else 0
     const int lane = threadIdx.x & 63;
-    const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int a = g < ncells ? cell_off[g] : 0, b = g < ncells ? cell_off[g + 1] : 0;
-    const int n = b - a;
-    // final place of the particle of cell-major position pos of cell gc
-    auto cluster = [&](int64_t gc, int &cs, int &cn) {
-        cs = 0;
-        cn = 0;
-        if (!cpc) return;
-        const int64_t cb = gc & ~(int64_t)(cpc - 1);
-        cs = cell_off[cb];
-        cn = cell_off[cb + cpc] - cs;
-    };
-    if (n > 0 && n <= kFixRegs) {
-        int cs, cn;
-        cluster(g, cs, cn);
-        auto put = [&](int pos, int32_t v) { dst[cpc ? cs + layout_slot(lay, pos - cs, cn) : pos] = v; };
-        if (n == 1) {
-            if (cpc) put(a, src[a]);
-        } else {
-            int ocs, ocn;
-            T.range(g, ocs, ocn);
-            int32_t v[kFixRegs];
-            uint64_t k[kFixRegs];
-#pragma unroll
-            for (int i = 0; i < kFixRegs; ++i) v[i] = i < n ? src[a + i] : 0;
-#pragma unroll
-            for (int i = 0; i < kFixRegs; ++i) k[i] = i < n ? fix_key(keys, T, v[i], ocs, ocn) : ~0ull;
-            bool sorted = true;
-#pragma unroll
-            for (int i = 1; i < kFixRegs; ++i) sorted &= k[i - 1] < k[i] || i >= n;
-            if (sorted) {
-                if (cpc)
-#pragma unroll
-                    for (int i = 0; i < kFixRegs; ++i)
-                        if (i < n) put(a + i, v[i]);
-            } else {
-#pragma unroll
-                for (int i = 0; i < kFixRegs; ++i) {
-                    int r = 0;
-#pragma unroll
-                    for (int j = 0; j < kFixRegs; ++j) r += k[j] < k[i] ? 1 : 0;
-                    if (i < n) put(a + r, v[i]);
-                }
-            }
+    const int64_t g = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * wcells + lane;
+    const bool mine = lane < wcells && g < ncells;
+    const int a = mine ? cell_off[g] : 0;
+    const int n = mine ? cell_off[g + 1] - a : 0;
+    // range of the lane's cluster, now and before
+    int cs = 0, cn = 0, ocs = 0, ocn = 0;
+    if (n > 0) {
+        if (cpc) {
+            const int64_t cb = g & ~(int64_t)(cpc - 1);
+            cs = cell_off[cb];
+            cn = cell_off[cb + cpc] - cs;
         }
-    }
-    if (!S.big) {
-        if (n <= kFixRegs) return;
-        int cs, cn, ocs, ocn;
-        cluster(g, cs, cn);
         T.range(g, ocs, ocn);
-        int32_t *perm = src;
-        for (int i = a + 1; i < b; ++i) {
-            const int32_t v = perm[i];
+    }
+    if (S.big) {
+        const int ib = wave_append(n > kFixMid, &S.nbig[0]);
+        if (n > kFixMid) S.big[ib] = (int32_t)g;
+    } else if (n > kFixMid) {
+        for (int i = a + 1; i < a + n; ++i) {
+            const int32_t v = src[i];
             const uint64_t kv = fix_key(keys, T, v, ocs, ocn);
             int j = i - 1;
             while (j >= a) {
-                const int32_t u = perm[j];
+                const int32_t u = src[j];
                 const uint64_t ku = fix_key(keys, T, u, ocs, ocn);
                 if (ku <= kv) break;
-                perm[j + 1] = u;
+                src[j + 1] = u;
                 --j;
             }
-            perm[j + 1] = v;
+            src[j + 1] = v;
         }
         if (cpc)
-            for (int i = a; i < b; ++i) dst[cs + layout_slot(lay, i - cs, cn)] = perm[i];
-        return;
+            for (int i = a; i < a + n; ++i) dst[cs + layout_slot(lay, i - cs, cn)] = src[i];
     }
-    const int ib = wave_append(n > kFixMid, &S.nbig[0]);
-    if (n > kFixMid) S.big[ib] = (int32_t)g;
-    // crowded cells of this wavefront's 64: pairs of up to 32 particles
-    const int64_t g0 = g - lane;
-    uint64_t half = __ballot(n > kFixRegs && n <= 32);
-    while (half) {
-        const int first = __ffsll((unsigned long long)half) - 1;
-        half &= half - 1;
-        const int second = half ? __ffsll((unsigned long long)half) - 1 : -1;
-        half &= half - 1;
-        const int mine = lane >= 32 ? second : first;  // this lane's cell, -1: none
-        const int l = lane & 31;
-        const int64_t gm = g0 + (mine < 0 ? first : mine);
-        const int am = cell_off[gm], nm = mine < 0 ? 0 : cell_off[gm + 1] - am;
-        int cs, cn, ocs, ocn;
-        cluster(gm, cs, cn);
-        T.range(gm, ocs, ocn);
-        const int32_t v = l < nm ? src[am + l] : 0;
-        const uint64_t k = l < nm ? fix_key(keys, T, v, ocs, ocn) : ~0ull;
-        const int n0 = __builtin_amdgcn_readlane(nm, 0), n1 = __builtin_amdgcn_readlane(nm, 32);
-        const int most = n0 > n1 ? n0 : n1;
-        int r = 0;
-        for (int j = 0; j < most; ++j) {  // places past a cell's end hold the largest key: never smaller
-            const uint64_t k0 = lane_key(k, j), k1 = lane_key(k, 32 + j);
-            r += (lane < 32 ? k0 : k1) < k ? 1 : 0;
-        }
-        if (l < nm) dst[cpc ? cs + layout_slot(lay, am + r - cs, cn) : am + r] = v;
+    // places of the lane's cell in the wavefront's run (in place, a single
+    // particle is where it belongs), and where they begin
+    const int m = n > kFixMid || (n == 1 && !cpc) ? 0 : n;
+    int end = m;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int e = __shfl_up(end, d, 64);
+        if (lane >= d) end += e;
     }
-    // and the others, up to kFixPer places per lane
-    uint64_t whole = __ballot(n > 32 && n <= kFixMid);
-    while (whole) {
-        const int64_t gm = g0 + (__ffsll((unsigned long long)whole) - 1);
-        whole &= whole - 1;
-        const int am = cell_off[gm], nm = __builtin_amdgcn_readfirstlane(cell_off[gm + 1] - am);
-        int cs, cn, ocs, ocn;
-        cluster(gm, cs, cn);
-        T.range(gm, ocs, ocn);
+    const int begin = end - m, total = __builtin_amdgcn_readlane(end, 63);
+    for (int base = 0; base < total;) {
+        // the cells that begin at base or later and end within the batch
+        const int len = __builtin_amdgcn_readlane(end, 63 - __builtin_clzll(__ballot(end - base <= kFixBatch))) - base;
+        static_assert(kFixBatch == 64 * 8, "a lane clears eight places");
+        *reinterpret_cast<uint64_t *>(sh + 8 * lane) = 0;
+        lds_order();
+        if (m > 0 && begin >= base && end - base <= len) sh[begin - base] = (uint8_t)(lane + 1);
+        lds_order();
         int32_t v[kFixPer];
-        uint64_t k[kFixPer];
-        int r[kFixPer];
+        int c[kFixPer];  // the lane that holds the place's cell
+        int last = 0;    // ... of the place before
 #pragma unroll
         for (int q = 0; q < kFixPer; ++q) {
-            const int l = lane + 64 * q;
-            r[q] = 0;
-            v[q] = l < nm ? src[am + l] : 0;
+            v[q] = 0;
+            c[q] = 0;
+            if (64 * q >= len) continue;
+            const int t = base + 64 * q + lane;
+            const int head = sh[64 * q + lane];
+            const uint64_t before = __ballot(head != 0) & (~0ull >> (63 - lane));
+            const int at = __shfl(head - 1, before ? 63 - __builtin_clzll(before) : lane, 64);
+            c[q] = before ? at : last;
+            last = __builtin_amdgcn_readlane(c[q], 63);
+            const int ac = __shfl(a - begin, c[q], 64);
+            if (t - base < len) v[q] = src[ac + t];
         }
 #pragma unroll
-        for (int q = 0; q < kFixPer; ++q) k[q] = lane + 64 * q < nm ? fix_key(keys, T, v[q], ocs, ocn) : ~0ull;
+        for (int q = 0; q < kFixPer; ++q) {
+            if (64 * q >= len) continue;
+            const int oc = __shfl(ocs, c[q], 64), on = __shfl(ocn, c[q], 64);
+            if (64 * q + lane < len) sk[64 * q + lane] = fix_key(keys, T, v[q], oc, on);
+        }
+        lds_order();
 #pragma unroll
         for (int q = 0; q < kFixPer; ++q) {
-            const int end = nm - 64 * q < 64 ? nm - 64 * q : 64;
-            for (int j = 0; j < end; ++j) {
-                const uint64_t kj = lane_key(k[q], j);
+            if (64 * q >= len) continue;
+            const int s = __shfl(begin, c[q], 64) - base, mc = __shfl(m, c[q], 64), ac = __shfl(a, c[q], 64);
+            const int ccs = __shfl(cs, c[q], 64), ccn = __shfl(cn, c[q], 64);
+            if (64 * q + lane < len) {
+                const uint64_t k = sk[64 * q + lane];
+                int r = ac;
+                for (int j = 0; j < mc; j += kFixAhead)
 #pragma unroll
-                for (int m = 0; m < kFixPer; ++m) r[m] += kj < k[m] ? 1 : 0;
+                    for (int i = 0; i < kFixAhead; ++i) r += j + i < mc && sk[s + j + i] < k ? 1 : 0;
+                dst[cpc ? ccs + layout_slot(lay, r - ccs, ccn) : r] = v[q];
             }
         }
-#pragma unroll
-        for (int q = 0; q < kFixPer; ++q)
-            if (lane + 64 * q < nm) dst[cpc ? cs + layout_slot(lay, am + r[q] - cs, cn) : am + r[q]] = v[q];
+        lds_order();
+        base += len;
     }
 }
 
@@ -747,7 +729,8 @@ void launch_sort(const Geom &g, const SortTask *tasks, int ns, hipStream_t st, b
                        in_cell_order ? 0 : cpc, layout, placed ? 1 : 0);
     SMI_LAUNCH_CHECK();
     if (!in_cell_order) return;
-    hipLaunchKernelGGL(k_bucket_fix, dim3(nblk(nc, 256), ns), dim3(256), 0, st, set, nc, cpc, layout, G);
+    const int wc = fix_cells(nc * ns);
+    hipLaunchKernelGGL(k_bucket_fix, dim3(nblk(nc, 4 * wc), ns), dim3(256), 0, st, set, nc, wc, cpc, layout, G);
     SMI_LAUNCH_CHECK();
     if (big) {
         hipLaunchKernelGGL(k_bucket_fix_big, dim3(big_blocks(most, nc), ns), dim3(kBigThreads), 0, st, set, cpc, layout, G);
