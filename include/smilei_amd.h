@@ -407,7 +407,9 @@ int smi_exchange_b(int ndim, int order, const int n_cells[3], const int patch_si
  * (may be NULL) the particles per patch, d_bin_index (may be NULL) per patch
  * the cumulative ends of its 4^3 (2D: 4^2) clusters relative to the patch's
  * first particle (Particles::last_index).  charge may be NULL; z may be
- * NULL in 2D.  Allocates its scratch; returns once the stream drained. */
+ * NULL in 2D.  Its scratch (20 bytes a particle, or up to 76 within 256 MiB, so
+ * that all arrays move together) comes from a pool of the device that keeps at
+ * most 256 MiB between calls; returns once the stream drained. */
 int smi_sort_exchange(int ndim, const int n_cells[3], const int patch_size[3], const double cell_length[3],
                       int64_t n, double *d_x, double *d_y, double *d_z, double *d_px, double *d_py, double *d_pz,
                       double *d_w, int16_t *d_charge, int32_t *d_key, int32_t *d_patch_count,

@@ -80,7 +80,8 @@ int smi_sort_exchange_noalloc(int ndim, const int n_cells[3], const int patch_si
                                                     std::to_string(kScratchWords));
     int32_t *base = scratch_ptr();
     if (!base) return SMI_ERR_HIP;
-    seams::SortScratch s = seams::carve_sort_scratch(g, n, base);
+    seams::SortScratch s =
+        seams::carve_sort_scratch(g, n, base, seams::sort_stage_arrays(g, n, kScratchWords));
     try {
         rc = seams::sort_exchange_impl(g, n, A, s, (hipStream_t)stream);
     } catch (const std::exception &e) {

@@ -21,7 +21,9 @@ int make_geom(int ndim, int order, const int n_cells[3], const int patch_size[3]
 struct SortScratch {
     SortBufs sb;
     uint32_t *keys;
-    double *stage;
+    double *stage;  // nstage arrays of stage_len doubles
+    int nstage;
+    int64_t stage_len;
     int *err;
 };
 
@@ -32,9 +34,14 @@ struct SortArrays {
 };
 
 // 4-byte words of scratch a sort/exchange of n particles over geometry g
-// needs, and its carving out of a buffer of that many words.
-int64_t sort_scratch_words(const Geom &g, int64_t n);
-SortScratch carve_sort_scratch(const Geom &g, int64_t n, int32_t *base);
+// needs with nstage particle arrays staged at a time (at least one), and its
+// carving out of a buffer of that many words.
+int64_t sort_scratch_words(const Geom &g, int64_t n, int nstage = 1);
+SortScratch carve_sort_scratch(const Geom &g, int64_t n, int32_t *base, int nstage = 1);
+
+// Particle arrays to stage at a time where the scratch may hold that many
+// words: all of them (eight, the charges as one) if they fit, one at least.
+int sort_stage_arrays(const Geom &g, int64_t n, int64_t words);
 
 // Checks of smi_sort_exchange's arguments; fills g.
 int sort_exchange_args(int ndim, const int n_cells[3], const int patch_size[3], const double cell_length[3],

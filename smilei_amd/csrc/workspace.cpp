@@ -9,7 +9,6 @@ namespace smi {
 
 namespace {
 
-constexpr uint64_t kKeep = 256ull << 20;  // bytes a pool holds between calls
 
 std::mutex g_lock;
 std::vector<hipMemPool_t> g_pool;  // by device; made at the first use, held until the process ends
@@ -25,7 +24,7 @@ hipMemPool_t device_pool(int dev)
         props.location.id = dev;
         hipMemPool_t pool = nullptr;
         if (hipMemPoolCreate(&pool, &props) != hipSuccess) return nullptr;
-        uint64_t keep = kKeep;
+        uint64_t keep = kWorkspaceKeep;
         (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
         g_pool[dev] = pool;
     }
