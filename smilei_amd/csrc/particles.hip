@@ -13,9 +13,9 @@
 //      (Projector{2D2,3D2,3D4}Order::currents) into an LDS tile with LDS
 //      FP64 atomics,
 //   3. flushes the J tile into the global arrays with FP64 atomics.
-// Gather, push and the per-particle current contributions use the
-// reference's association order (the file is built with -ffp-contract=off),
-// so only the order of the J summation differs from the CPU operators.
+// Without DEPOSIT, gather and push use the reference's association order (the
+// file is built with -ffp-contract=off); with it they are factorised and
+// fused, as the current contributions are.
 //
 // k_det_deposit{3,2}: the same current contributions added in the reference's
 // order into per-patch ghosted arrays; then the J ghost sum in x, y, z passes
@@ -276,26 +276,33 @@ __device__ __attribute__((always_inline)) inline void fp_cluster(const Geom &g, 
             }
             continue;
         }
+        // DEPOSIT (the atomic form, whose sums have no fixed order): the fused
+        // gather and push; else the reference's association order, bit for bit
         double Ep[3], Bp[3];
-        if constexpr (ND == 3) {
-            Ep[0] = gather3<H, GT, GSX>(cd[0], cp[1], cp[2], sF + 0 * GF, ld[0], lp[1], lp[2]);
-            Ep[1] = gather3<H, GT, GSX>(cp[0], cd[1], cp[2], sF + 1 * GF, lp[0], ld[1], lp[2]);
-            Ep[2] = gather3<H, GT, GSX>(cp[0], cp[1], cd[2], sF + 2 * GF, lp[0], lp[1], ld[2]);
-            Bp[0] = gather3<H, GT, GSX>(cp[0], cd[1], cd[2], sF + 3 * GF, lp[0], ld[1], ld[2]);
-            Bp[1] = gather3<H, GT, GSX>(cd[0], cp[1], cd[2], sF + 4 * GF, ld[0], lp[1], ld[2]);
-            Bp[2] = gather3<H, GT, GSX>(cd[0], cd[1], cp[2], sF + 5 * GF, ld[0], ld[1], lp[2]);
-        } else {
-            Ep[0] = gather2<H, GT>(cd[0], cp[1], sF + 0 * GF, ld[0], lp[1]);
-            Ep[1] = gather2<H, GT>(cp[0], cd[1], sF + 1 * GF, lp[0], ld[1]);
-            Ep[2] = gather2<H, GT>(cp[0], cp[1], sF + 2 * GF, lp[0], lp[1]);
-            Bp[0] = gather2<H, GT>(cp[0], cd[1], sF + 3 * GF, lp[0], ld[1]);
-            Bp[1] = gather2<H, GT>(cd[0], cp[1], sF + 4 * GF, ld[0], lp[1]);
-            Bp[2] = gather2<H, GT>(cd[0], cd[1], sF + 5 * GF, ld[0], ld[1]);
-        }
+        auto gather = [&](int f, int dual) {
+            const double *c[3];
+            int l[3];
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                c[d] = (dual >> d) & 1 ? cd[d] : cp[d];
+                l[d] = (dual >> d) & 1 ? ld[d] : lp[d];
+            }
+            if constexpr (ND == 3 && DEPOSIT) return gather3_fused<H, GT, GSX>(c[0], c[1], c[2], sF + f * GF, l[0], l[1], l[2]);
+            else if constexpr (ND == 3) return gather3<H, GT, GSX>(c[0], c[1], c[2], sF + f * GF, l[0], l[1], l[2]);
+            else if constexpr (DEPOSIT) return gather2_fused<H, GT>(c[0], c[1], sF + f * GF, l[0], l[1]);
+            else return gather2<H, GT>(c[0], c[1], sF + f * GF, l[0], l[1]);
+        };
+        Ep[0] = gather(0, 1);
+        Ep[1] = gather(1, 2);
+        Ep[2] = gather(2, 4);
+        Bp[0] = gather(3, 6);
+        Bp[1] = gather(4, 5);
+        Bp[2] = gather(5, 3);
 
         // ---- push
         double dxp[3], invgf;
-        boris(sp.qmh, g.dt, Ep, Bp, u, dxp, invgf);
+        if constexpr (DEPOSIT) boris_fused(sp.qmh, g.dt, Ep, Bp, u, dxp, invgf);
+        else boris(sp.qmh, g.dt, Ep, Bp, u, dxp, invgf);
         double xn[3];
 #pragma unroll
         for (int d = 0; d < ND; ++d) xn[d] = x[d] + dxp[d];

@@ -234,6 +234,84 @@ __device__ inline double gather2(const double *cx, const double *cy, const doubl
     return r;
 }
 
+// The same sums factorised by axis and fused: one FMA per point and one per
+// row and plane, 39 operations at order 2 and 155 at order 4 against 90 and
+// 400.  Rounded less often than the forms above, and not as they are.
+template <int H, int T, int SX = T * T>
+__device__ inline double gather3_fused(const double *cx, const double *cy, const double *cz, const double *t, int i,
+                                       int j, int k)
+{
+    double r = 0.;
+#pragma unroll
+    for (int a = -H; a <= H; ++a) {
+        double p = 0.;
+#pragma unroll
+        for (int b = -H; b <= H; ++b) {
+            double q = 0.;
+#pragma unroll
+            for (int c = -H; c <= H; ++c) q = fma(cz[c + H], t[(i + a) * SX + (j + b) * T + (k + c)], q);
+            p = fma(cy[b + H], q, p);
+        }
+        r = fma(cx[a + H], p, r);
+    }
+    return r;
+}
+
+template <int H, int T>
+__device__ inline double gather2_fused(const double *cx, const double *cy, const double *t, int i, int j)
+{
+    double r = 0.;
+#pragma unroll
+    for (int a = -H; a <= H; ++a) {
+        double p = 0.;
+#pragma unroll
+        for (int b = -H; b <= H; ++b) p = fma(cy[b + H], t[(i + a) * T + (j + b)], p);
+        r = fma(cx[a + H], p, r);
+    }
+    return r;
+}
+
+// 1/x and 1/sqrt(x) for x >= 1 to about one unit in the last place: the
+// hardware's estimate (24 bits and more) and one third-order step, whose error
+// is the cube of the estimate's.
+__device__ inline double rcp_cubic(double x)
+{
+    const double y = __builtin_amdgcn_rcp(x), e = fma(-x, y, 1.);
+    return fma(y, fma(e, e, e), y);
+}
+
+__device__ inline double rsqrt_cubic(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x), e = fma(-x * y, y, 1.);
+    return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// Boris push by the two cross products, fused.  The last factor, 1/gamma of
+// the new momentum, is rounded as boris() rounds it, so without fields the two
+// agree bit for bit.
+__device__ inline void boris_fused(double qmh, double dt, const double *E, const double *B, double *u, double *dxp,
+                                   double &invgf)
+{
+    const double ux = fma(qmh, E[0], u[0]), uy = fma(qmh, E[1], u[1]), uz = fma(qmh, E[2], u[2]);
+    const double f = qmh * rsqrt_cubic(fma(ux, ux, fma(uy, uy, fma(uz, uz, 1.))));
+    const double tx = f * B[0], ty = f * B[1], tz = f * B[2];
+    const double s = 2. * rcp_cubic(fma(tx, tx, fma(ty, ty, fma(tz, tz, 1.))));
+    const double vx = fma(uy, tz, fma(-uz, ty, ux)), vy = fma(uz, tx, fma(-ux, tz, uy)),
+                 vz = fma(ux, ty, fma(-uy, tx, uz));
+    const double sx = s * tx, sy = s * ty, sz = s * tz;
+    const double ax = fma(qmh, E[0], fma(vy, sz, fma(-vz, sy, ux))), ay = fma(qmh, E[1], fma(vz, sx, fma(-vx, sz, uy))),
+                 az = fma(qmh, E[2], fma(vx, sy, fma(-vy, sx, uz)));
+    double gi = 1. / sqrt(1.0 + ax * ax + ay * ay + az * az);
+    invgf = gi;
+    u[0] = ax;
+    u[1] = ay;
+    u[2] = az;
+    gi *= dt;
+    dxp[0] = ax * gi;
+    dxp[1] = ay * gi;
+    dxp[2] = az * gi;
+}
+
 // Same gathers on a strided array (the reference's per-patch Field3D/2D).
 // O: unsigned 32-bit byte offsets from the array's scalar base where the array
 // is below 4 GiB, one add per row; 64-bit ones otherwise.
