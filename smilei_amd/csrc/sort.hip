@@ -163,11 +163,9 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(SortSet set, int64_
     }
     const int64_t base = (int64_t)blockIdx.x * kScanTile + (int64_t)threadIdx.x * kScanItems;
     const bool full = (int64_t)(blockIdx.x + 1) * kScanTile <= n;
-    if (clus_old) {
-#pragma unroll
-        for (int k = 0; k < kScanItems; ++k)
-            if (base + k < n && (base + k) % cpcell == 0) clus_old[(base + k) / cpcell] = out[base + k];
-    }
+    // (a cluster is 16 or 64 cells: it begins at the first of a thread's
+    // entries if at any)
+    if (clus_old && base < n && (base & (cpcell - 1)) == 0) clus_old[base >> __builtin_ctz(cpcell)] = out[base];
     int v[kScanItems];
     int s = 0;
     if (full) {
@@ -359,7 +357,7 @@ struct TieSrc {
         cs = 0;
         cn = 0;
         if (!tie || !clus_old) return;
-        const int b = (int)(g / cpcell);
+        const int b = (int)g >> __builtin_ctz(cpcell);  // 16 or 64 cells; fewer than 2^27 in all
         cs = clus_old[b];
         cn = (b + 1 < ncl ? clus_old[b + 1] : (int)n) - cs;
     }
