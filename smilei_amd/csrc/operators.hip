@@ -191,11 +191,19 @@ __global__ void __launch_bounds__(128, 2) k_proj3d_atomic(Proj3Args a)
 // two to a bank pair.
 // Binning pays from this many particles on.  Sorted / unsorted arrays,
 // microseconds, per-particle atomics against bins: order 2, 4,096 particles
-// 20 / 31 against 41 / 41, 8,192 29 / 48 against 40 / 39, 32,768 88 / 160
-// against 45 / 54, 2.1e6 4,000 / 7,222 against 307 / 548; order 4, 512
-// particles 54 / 79 against 38 / 40, 32,768 432 / 775 against 88 / 87, 2.1e6
-// 19,020 / 34,860 against 973 / 753.
-constexpr int64_t bin_min(int order) { return order == 2 ? 12288 : 512; }
+// 20 / 31 against 22 / 22, 8,192 29 / 47 against 23 / 23, 32,768 88 / 160
+// against 39 / 40, 2.1e6 4,000 / 7,222 against 211 / 473; order 4, 64
+// particles 39 / 40 against 24 / 23, 512 54 / 79 against 24 / 24, 32,768 432 /
+// 775 against 79 / 64, 2.1e6 19,020 / 34,860 against 907 / 666.
+constexpr int64_t bin_min(int order) { return order == 2 ? 8192 : 64; }
+
+// Up to this many particles one workgroup does all of the binning: four
+// launches less against the work of one CU.  Whole call, one workgroup against
+// many (sorted / unsorted): order 2, 8,192 particles 23 / 23 against 37 / 36,
+// 12,288 27 / 28 against 37 / 36, 16,384 32 / 34 against 40 / 36, 32,768 49 / 55
+// against 39 / 40; order 4, 64 particles 24 against 35, 12,288 46 / 44 against
+// 45 / 42, 16,384 58 / 56 against 54 / 49.
+constexpr int64_t bin_one_max(int order) { return order == 2 ? 12288 : 8192; }
 
 template <int ORDER>
 struct BinTile {
@@ -226,7 +234,8 @@ __device__ inline int node_bin(const Proj3Args &a, const Bins &b, int64_t i)
 }
 
 // Bin and place in the bin of every particle.  Lanes of a wavefront with
-// equal bins in a row (particles in cell order) share one atomic.
+// equal bins in a row (particles in cell order) share one atomic.  For more
+// bins than a workgroup counts in LDS.
 template <int ORDER>
 __global__ void __launch_bounds__(256) k_bin_count(Proj3Args a, Bins b)
 {
@@ -241,6 +250,89 @@ __global__ void __launch_bounds__(256) k_bin_count(Proj3Args a, Bins b)
     if (i < a.n) {
         b.key[i] = key;
         b.rank[i] = first + lane - head;
+    }
+}
+
+// The same counted in LDS first, `per` particles a thread, and added to the
+// bins' counts by one atomic per workgroup and bin: the atomics of one bin
+// queue up otherwise (order 2, whole call, with k_bin_count: 2.6e5 particles
+// 88 us in cell order and 131 shuffled, here 56 and 69; 2.1e6 307 and 558, here
+// 211 and 473).
+constexpr int kBinLds = 8192, kBinThreads = 1024;
+
+template <int ORDER>
+__device__ inline void bin_count_lds(const Proj3Args &a, const Bins &b, int nbins, int64_t i0, int per, int *h)
+{
+    for (int q = threadIdx.x; q < nbins; q += kBinThreads) h[q] = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+#pragma unroll 4
+    for (int k = 0; k < per; ++k) {
+        const int64_t i = i0 + (int64_t)k * kBinThreads + threadIdx.x;
+        const int key = i < a.n ? node_bin<ORDER>(a, b, i) : -1;
+        int head, len;
+        key_run((uint32_t)key, head, len);
+        int first = 0;
+        if (lane == head && key >= 0) first = atomicAdd(&h[key], len);
+        first = __shfl(first, head, 64);
+        if (i < a.n) {
+            b.key[i] = key;
+            b.rank[i] = first + lane - head;
+        }
+    }
+    __syncthreads();
+}
+
+template <int ORDER>
+__global__ void __launch_bounds__(kBinThreads) k_bin_count_lds(Proj3Args a, Bins b, int nbins, int per)
+{
+    __shared__ int h[kBinLds];
+    const int64_t i0 = (int64_t)blockIdx.x * per * kBinThreads;
+    bin_count_lds<ORDER>(a, b, nbins, i0, per, h);
+#pragma unroll 4
+    for (int q = threadIdx.x; q < nbins; q += kBinThreads)
+        if (h[q]) h[q] = atomicAdd(&b.count[q], h[q]);
+    __syncthreads();
+#pragma unroll 4
+    for (int k = 0; k < per; ++k) {
+        const int64_t i = i0 + (int64_t)k * kBinThreads + threadIdx.x;
+        if (i < a.n && b.key[i] >= 0) b.rank[i] += h[b.key[i]];
+    }
+}
+
+// All of the binning by one workgroup: count, start of the bins and list, one
+// launch instead of four.
+template <int ORDER>
+__global__ void __launch_bounds__(kBinThreads) k_bin_one(Proj3Args a, Bins b, int nbins, int per)
+{
+    __shared__ int h[kBinLds];
+    __shared__ int part[kBinThreads / 64];
+    bin_count_lds<ORDER>(a, b, nbins, 0, per, h);
+    const int run = (nbins + kBinThreads - 1) / kBinThreads, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int q0 = threadIdx.x * run, q1 = q0 + run < nbins ? q0 + run : nbins;
+    int sum = 0;
+    for (int q = q0; q < q1; ++q) sum += h[q];
+    int incl = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += t;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    int at = incl - sum;
+    for (int w = 0; w < wave; ++w) at += part[w];
+    for (int q = q0; q < q1; ++q) {
+        const int c = h[q];
+        b.start[q] = h[q] = at;
+        at += c;
+    }
+    if (threadIdx.x == kBinThreads - 1) b.start[nbins] = at;
+    __syncthreads();
+#pragma unroll 4
+    for (int k = 0; k < per; ++k) {
+        const int64_t i = (int64_t)k * kBinThreads + threadIdx.x;
+        if (i < a.n && b.key[i] >= 0) b.list[h[b.key[i]] + b.rank[i]] = (int)i;
     }
 }
 
@@ -562,12 +654,29 @@ bool launch_bins(int order, const Proj3Args &a, hipStream_t st)
     b.key = b.start + nbins + 1;
     b.rank = b.key + a.n;
     b.list = b.rank + a.n;
-    launch_fill_i32(b.count, nbins, 0, st);
-    const dim3 per(nblk(a.n, 256)), block(256);
-    if (order == 2) hipLaunchKernelGGL(k_bin_count<2>, per, block, 0, st, a, b);
-    else hipLaunchKernelGGL(k_bin_count<4>, per, block, 0, st, a, b);
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, st, b, (int)nbins);
-    hipLaunchKernelGGL(k_bin_fill, per, block, 0, st, b, a.n);
+    const dim3 block(256);
+    if (nbins <= kBinLds && a.n <= bin_one_max(order)) {
+        const int per = (int)nblk(a.n, kBinThreads);
+        if (order == 2) hipLaunchKernelGGL(k_bin_one<2>, dim3(1), dim3(kBinThreads), 0, st, a, b, (int)nbins, per);
+        else hipLaunchKernelGGL(k_bin_one<4>, dim3(1), dim3(kBinThreads), 0, st, a, b, (int)nbins, per);
+    } else {
+        launch_fill_i32(b.count, nbins, 0, st);
+        if (nbins <= kBinLds) {
+            // a workgroup per CU where there are that many particles, 16
+            // particles a thread at most, and half a bin's worth a thread at
+            // least, as the bins are cleared and added up once per workgroup
+            const int64_t want = std::max<int64_t>(a.n / (256 * kBinThreads), nbins / (2 * kBinThreads));
+            const int per = (int)std::min<int64_t>(std::max<int64_t>(want, 1), 16);
+            const dim3 grid(nblk(a.n, (int64_t)per * kBinThreads)), wide(kBinThreads);
+            if (order == 2) hipLaunchKernelGGL(k_bin_count_lds<2>, grid, wide, 0, st, a, b, (int)nbins, per);
+            else hipLaunchKernelGGL(k_bin_count_lds<4>, grid, wide, 0, st, a, b, (int)nbins, per);
+        } else {
+            if (order == 2) hipLaunchKernelGGL(k_bin_count<2>, dim3(nblk(a.n, 256)), block, 0, st, a, b);
+            else hipLaunchKernelGGL(k_bin_count<4>, dim3(nblk(a.n, 256)), block, 0, st, a, b);
+        }
+        hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, st, b, (int)nbins);
+        hipLaunchKernelGGL(k_bin_fill, dim3(nblk(a.n, 256)), block, 0, st, b, a.n);
+    }
     if (order == 2) hipLaunchKernelGGL(k_proj3d_bins<2>, dim3((unsigned)nbins), block, 0, st, a, b);
     else hipLaunchKernelGGL(k_proj3d_bins<4>, dim3((unsigned)nbins), block, 0, st, a, b);
     return true;
