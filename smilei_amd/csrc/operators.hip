@@ -217,9 +217,17 @@ struct Bins {
     int *key, *rank, *list;  // per particle
 };
 
-// Bin of particle i, or -1 for one whose stencil would leave the arrays.
+// Bin of particle i by its old node, or -1 for one whose stencil would leave
+// the arrays.
 template <int ORDER>
-__device__ inline int node_bin(const Proj3Args &a, const Bins &b, int64_t i)
+struct NodeKey {
+    Proj3Args a;
+    __device__ int64_t n() const { return a.n; }
+    __device__ int operator()(const Bins &b, int64_t i) const;
+};
+
+template <int ORDER>
+__device__ inline int NodeKey<ORDER>::operator()(const Bins &b, int64_t i) const
 {
     constexpr int H = ORDER / 2;
     int key = 0;
@@ -236,18 +244,18 @@ __device__ inline int node_bin(const Proj3Args &a, const Bins &b, int64_t i)
 // Bin and place in the bin of every particle.  Lanes of a wavefront with
 // equal bins in a row (particles in cell order) share one atomic.  For more
 // bins than a workgroup counts in LDS.
-template <int ORDER>
-__global__ void __launch_bounds__(256) k_bin_count(Proj3Args a, Bins b)
+template <class Key>
+__global__ void __launch_bounds__(256) k_bin_count(Key of, Bins b)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63;
-    const int key = i < a.n ? node_bin<ORDER>(a, b, i) : -1;
+    const int key = i < of.n() ? of(b, i) : -1;
     int head, len;
     key_run((uint32_t)key, head, len);
     int first = 0;
     if (lane == head && key >= 0) first = atomicAdd(&b.count[key], len);
     first = __shfl(first, head, 64);
-    if (i < a.n) {
+    if (i < of.n()) {
         b.key[i] = key;
         b.rank[i] = first + lane - head;
     }
@@ -260,8 +268,8 @@ __global__ void __launch_bounds__(256) k_bin_count(Proj3Args a, Bins b)
 // 211 and 473).
 constexpr int kBinLds = 8192, kBinThreads = 1024;
 
-template <int ORDER>
-__device__ inline void bin_count_lds(const Proj3Args &a, const Bins &b, int nbins, int64_t i0, int per, int *h)
+template <class Key>
+__device__ inline void bin_count_lds(const Key &of, const Bins &b, int nbins, int64_t i0, int per, int *h)
 {
     for (int q = threadIdx.x; q < nbins; q += kBinThreads) h[q] = 0;
     __syncthreads();
@@ -269,13 +277,13 @@ __device__ inline void bin_count_lds(const Proj3Args &a, const Bins &b, int nbin
 #pragma unroll 4
     for (int k = 0; k < per; ++k) {
         const int64_t i = i0 + (int64_t)k * kBinThreads + threadIdx.x;
-        const int key = i < a.n ? node_bin<ORDER>(a, b, i) : -1;
+        const int key = i < of.n() ? of(b, i) : -1;
         int head, len;
         key_run((uint32_t)key, head, len);
         int first = 0;
         if (lane == head && key >= 0) first = atomicAdd(&h[key], len);
         first = __shfl(first, head, 64);
-        if (i < a.n) {
+        if (i < of.n()) {
             b.key[i] = key;
             b.rank[i] = first + lane - head;
         }
@@ -283,12 +291,12 @@ __device__ inline void bin_count_lds(const Proj3Args &a, const Bins &b, int nbin
     __syncthreads();
 }
 
-template <int ORDER>
-__global__ void __launch_bounds__(kBinThreads) k_bin_count_lds(Proj3Args a, Bins b, int nbins, int per)
+template <class Key>
+__global__ void __launch_bounds__(kBinThreads) k_bin_count_lds(Key of, Bins b, int nbins, int per)
 {
     __shared__ int h[kBinLds];
     const int64_t i0 = (int64_t)blockIdx.x * per * kBinThreads;
-    bin_count_lds<ORDER>(a, b, nbins, i0, per, h);
+    bin_count_lds(of, b, nbins, i0, per, h);
 #pragma unroll 4
     for (int q = threadIdx.x; q < nbins; q += kBinThreads)
         if (h[q]) h[q] = atomicAdd(&b.count[q], h[q]);
@@ -296,18 +304,18 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_count_lds(Proj3Args a, Bins
 #pragma unroll 4
     for (int k = 0; k < per; ++k) {
         const int64_t i = i0 + (int64_t)k * kBinThreads + threadIdx.x;
-        if (i < a.n && b.key[i] >= 0) b.rank[i] += h[b.key[i]];
+        if (i < of.n() && b.key[i] >= 0) b.rank[i] += h[b.key[i]];
     }
 }
 
 // All of the binning by one workgroup: count, start of the bins and list, one
 // launch instead of four.
-template <int ORDER>
-__global__ void __launch_bounds__(kBinThreads) k_bin_one(Proj3Args a, Bins b, int nbins, int per)
+template <class Key>
+__global__ void __launch_bounds__(kBinThreads) k_bin_one(Key of, Bins b, int nbins, int per)
 {
     __shared__ int h[kBinLds];
     __shared__ int part[kBinThreads / 64];
-    bin_count_lds<ORDER>(a, b, nbins, 0, per, h);
+    bin_count_lds(of, b, nbins, 0, per, h);
     const int run = (nbins + kBinThreads - 1) / kBinThreads, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int q0 = threadIdx.x * run, q1 = q0 + run < nbins ? q0 + run : nbins;
     int sum = 0;
@@ -332,7 +340,7 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_one(Proj3Args a, Bins b, in
 #pragma unroll 4
     for (int k = 0; k < per; ++k) {
         const int64_t i = (int64_t)k * kBinThreads + threadIdx.x;
-        if (i < a.n && b.key[i] >= 0) b.list[h[b.key[i]] + b.rank[i]] = (int)i;
+        if (i < of.n() && b.key[i] >= 0) b.list[h[b.key[i]] + b.rank[i]] = (int)i;
     }
 }
 
@@ -637,6 +645,37 @@ int op_fail(int code, const std::string &m)
 
 // The binned projection where it is the faster one and has its scratch;
 // false otherwise.
+int64_t bins_words(int64_t nbins, int64_t n) { return 2 * nbins + 1 + 3 * n; }
+
+// Lists the n particles by bin: b.start and b.list, in ws (bins_words).
+template <class Key>
+void launch_binning(const Key &of, Bins &b, int64_t nbins, int64_t n, int64_t one_max, int *ws, hipStream_t st)
+{
+    b.count = ws;
+    b.start = b.count + nbins;
+    b.key = b.start + nbins + 1;
+    b.rank = b.key + n;
+    b.list = b.rank + n;
+    const dim3 wide(kBinThreads);
+    if (nbins <= kBinLds && n <= one_max) {
+        hipLaunchKernelGGL(k_bin_one<Key>, dim3(1), wide, 0, st, of, b, (int)nbins, (int)nblk(n, kBinThreads));
+        return;
+    }
+    launch_fill_i32(b.count, nbins, 0, st);
+    if (nbins <= kBinLds) {
+        // a workgroup per CU where there are that many particles, 16 particles
+        // a thread at most, and half a bin's worth a thread at least, as the
+        // bins are cleared and added up once per workgroup
+        const int64_t want = std::max<int64_t>(n / (256 * kBinThreads), nbins / (2 * kBinThreads));
+        const int per = (int)std::min<int64_t>(std::max<int64_t>(want, 1), 16);
+        hipLaunchKernelGGL(k_bin_count_lds<Key>, dim3(nblk(n, per * kBinThreads)), wide, 0, st, of, b, (int)nbins, per);
+    } else {
+        hipLaunchKernelGGL(k_bin_count<Key>, dim3(nblk(n, 256)), dim3(256), 0, st, of, b);
+    }
+    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, st, b, (int)nbins);
+    hipLaunchKernelGGL(k_bin_fill, dim3(nblk(n, 256)), dim3(256), 0, st, b, n);
+}
+
 bool launch_bins(int order, const Proj3Args &a, hipStream_t st)
 {
     if (a.n < bin_min(order) || a.n >= (1ll << 31)) return false;
@@ -647,38 +686,141 @@ bool launch_bins(int order, const Proj3Args &a, hipStream_t st)
         nbins *= b.nb[d];
     }
     if (nbins > a.n) return false;  // less than one particle per bin
-    const Workspace ws((size_t)(2 * nbins + 1 + 3 * a.n) * sizeof(int), st);
+    const Workspace ws((size_t)bins_words(nbins, a.n) * sizeof(int), st);
     if (!ws.p) return false;
-    b.count = (int *)ws.p;
-    b.start = b.count + nbins;
-    b.key = b.start + nbins + 1;
-    b.rank = b.key + a.n;
-    b.list = b.rank + a.n;
     const dim3 block(256);
-    if (nbins <= kBinLds && a.n <= bin_one_max(order)) {
-        const int per = (int)nblk(a.n, kBinThreads);
-        if (order == 2) hipLaunchKernelGGL(k_bin_one<2>, dim3(1), dim3(kBinThreads), 0, st, a, b, (int)nbins, per);
-        else hipLaunchKernelGGL(k_bin_one<4>, dim3(1), dim3(kBinThreads), 0, st, a, b, (int)nbins, per);
+    if (order == 2) {
+        launch_binning(NodeKey<2>{a}, b, nbins, a.n, bin_one_max(2), (int *)ws.p, st);
+        hipLaunchKernelGGL(k_proj3d_bins<2>, dim3((unsigned)nbins), block, 0, st, a, b);
     } else {
-        launch_fill_i32(b.count, nbins, 0, st);
-        if (nbins <= kBinLds) {
-            // a workgroup per CU where there are that many particles, 16
-            // particles a thread at most, and half a bin's worth a thread at
-            // least, as the bins are cleared and added up once per workgroup
-            const int64_t want = std::max<int64_t>(a.n / (256 * kBinThreads), nbins / (2 * kBinThreads));
-            const int per = (int)std::min<int64_t>(std::max<int64_t>(want, 1), 16);
-            const dim3 grid(nblk(a.n, (int64_t)per * kBinThreads)), wide(kBinThreads);
-            if (order == 2) hipLaunchKernelGGL(k_bin_count_lds<2>, grid, wide, 0, st, a, b, (int)nbins, per);
-            else hipLaunchKernelGGL(k_bin_count_lds<4>, grid, wide, 0, st, a, b, (int)nbins, per);
-        } else {
-            if (order == 2) hipLaunchKernelGGL(k_bin_count<2>, dim3(nblk(a.n, 256)), block, 0, st, a, b);
-            else hipLaunchKernelGGL(k_bin_count<4>, dim3(nblk(a.n, 256)), block, 0, st, a, b);
-        }
-        hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, st, b, (int)nbins);
-        hipLaunchKernelGGL(k_bin_fill, dim3(nblk(a.n, 256)), block, 0, st, b, a.n);
+        launch_binning(NodeKey<4>{a}, b, nbins, a.n, bin_one_max(4), (int *)ws.p, st);
+        hipLaunchKernelGGL(k_proj3d_bins<4>, dim3((unsigned)nbins), block, 0, st, a, b);
     }
-    if (order == 2) hipLaunchKernelGGL(k_proj3d_bins<2>, dim3((unsigned)nbins), block, 0, st, a, b);
-    else hipLaunchKernelGGL(k_proj3d_bins<4>, dim3((unsigned)nbins), block, 0, st, a, b);
+    return true;
+}
+
+// Interpolation of particles binned by node: a bin's particles gather from a
+// tile of the six fields in LDS (5 + 2H points per axis), by the same
+// products and sums as k_interp3d, so to the same bits.  Gathered from global
+// memory, a particle's rows come through the L1 (64 bytes a clock, half of what
+// LDS gives) while its neighbours are near it, and through the L2 when the
+// array is in no order.  The gathers are kept apart (scheduling barriers): 23
+// registers spilled at three wavefronts per SIMD, 415 us for 2.1e6 particles
+// against 438 without, and against 439 with two wavefronts and no spills.
+struct Interp3Args {
+    const double *F[6];  // Ex, Ey, Ez, Bx, By, Bz
+    Ints3 np, dom;
+    Dbl3 dinv;
+    int64_t n;
+    const double *x[3];
+    double *Ep, *Bp;
+    int32_t *iold;
+    double *dold;
+};
+
+// Bin of particle i by its node; -1, and NaN as its result, for one outside
+// the patch.
+template <int ORDER>
+struct PlaceKey {
+    Interp3Args a;
+    __device__ int64_t n() const { return a.n; }
+    __device__ int operator()(const Bins &b, int64_t i) const
+    {
+        constexpr int H = ORDER / 2;
+        int key = 0;
+        bool ok = true;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double pn = a.x[d][i] * a.dinv.v[d];
+            const int ip = (int)round(pn) - a.dom.v[d], id = (int)round(pn + 0.5) - a.dom.v[d];
+            ok &= ip >= H && ip + H <= a.np.v[d] - 1 && id >= H && id + H <= a.np.v[d];
+            key = key * b.nb[d] + (ip >> 2);
+        }
+        if (!ok)
+            for (int c = 0; c < 3; ++c) a.Ep[c * a.n + i] = a.Bp[c * a.n + i] = __builtin_nan("");
+        return ok ? key : -1;
+    }
+};
+
+template <int ORDER>
+__global__ void __launch_bounds__(256, 3) k_interp3d_bins(Interp3Args a, Bins b)
+{
+    constexpr int H = ORDER / 2, T = 5 + 2 * H, SY = T, SX = T * T + 3, SF = T * SX;
+    __shared__ double s[6 * SF];
+    const int bin = blockIdx.x, first = b.start[bin], last = b.start[bin + 1];
+    if (first == last) return;
+    // tile point 0 is point 4 q - H of an axis; points outside an array are read by no particle of the bin
+    const int q[3] = {bin / (b.nb[1] * b.nb[2]) * 4 - H, bin / b.nb[2] % b.nb[1] * 4 - H, bin % b.nb[2] * 4 - H};
+    for (int t = threadIdx.x; t < T * T * T; t += blockDim.x) {
+        const int l[3] = {t / (T * T), t / T % T, t % T};
+#pragma unroll
+        for (int f = 0; f < 6; ++f) {
+            bool in = true;
+            int64_t idx = 0;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                const int m = a.np.v[d] + ((f < 3) == (f % 3 == d) ? 1 : 0), g = q[d] + l[d];
+                in &= g >= 0 && g < m;
+                idx = idx * m + g;
+            }
+            s[f * SF + l[0] * SX + l[1] * SY + l[2]] = in ? a.F[f][idx] : 0.;
+        }
+    }
+    __syncthreads();
+    for (int t = first + threadIdx.x; t < last; t += blockDim.x) {
+        const int64_t i = b.list[t];
+        double cp[3][5], cd[3][5];
+        int lp[3], ld[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const double pn = a.x[d][i] * a.dinv.v[d];
+            int ip = (int)round(pn), id = (int)round(pn + 0.5);
+            const double dp = pn - (double)ip;
+            spline<ORDER>(dp, cp[d]);
+            spline<ORDER>(pn - (double)id + 0.5, cd[d]);
+            ip -= a.dom.v[d];
+            id -= a.dom.v[d];
+            lp[d] = ip - q[d];
+            ld[d] = id - q[d];
+            a.iold[d * a.n + i] = ip;
+            a.dold[d * a.n + i] = dp;
+        }
+        a.Ep[i] = gather3<H, SY, SX>(cd[0], cp[1], cp[2], s + 0 * SF, ld[0], lp[1], lp[2]);
+        __builtin_amdgcn_sched_barrier(0);
+        a.Ep[a.n + i] = gather3<H, SY, SX>(cp[0], cd[1], cp[2], s + 1 * SF, lp[0], ld[1], lp[2]);
+        __builtin_amdgcn_sched_barrier(0);
+        a.Ep[2 * a.n + i] = gather3<H, SY, SX>(cp[0], cp[1], cd[2], s + 2 * SF, lp[0], lp[1], ld[2]);
+        __builtin_amdgcn_sched_barrier(0);
+        a.Bp[i] = gather3<H, SY, SX>(cp[0], cd[1], cd[2], s + 3 * SF, lp[0], ld[1], ld[2]);
+        __builtin_amdgcn_sched_barrier(0);
+        a.Bp[a.n + i] = gather3<H, SY, SX>(cd[0], cp[1], cd[2], s + 4 * SF, ld[0], lp[1], ld[2]);
+        __builtin_amdgcn_sched_barrier(0);
+        a.Bp[2 * a.n + i] = gather3<H, SY, SX>(cd[0], cd[1], cp[2], s + 5 * SF, ld[0], ld[1], lp[2]);
+    }
+}
+
+// Where binning pays: order 4, this many particles, and so many to a bin (the
+// tile of a bin is 9^3 points of six fields).  Whole call, cell order / no order,
+// k_interp3d against bins: 2.6e5 particles 83 / 205 us against 95 / 142; 5.1e5 159
+// / 455 against 146 / 220; 1.0e6, 180 to a bin, 282 / 1,733 against 261 / 378;
+// 2.1e6 524 / 4,002 against 415 / 853; but 5.2e5, 90 to a bin, 143 against 195 in
+// cell order.  Order 2, 2.1e6: 144 / 886 against 166 / 466, left as it is.
+constexpr int64_t kInterpBinMin = 1 << 19, kInterpPerBin = 160;
+
+bool launch_interp_bins(int order, const Interp3Args &a, hipStream_t st)
+{
+    if (order != 4 || a.n < kInterpBinMin || a.n >= (1ll << 31)) return false;
+    Bins b{};
+    int64_t nbins = 1;
+    for (int d = 0; d < 3; ++d) {
+        b.nb[d] = (a.np.v[d] + 3) / 4;
+        nbins *= b.nb[d];
+    }
+    if (nbins < 1 || a.n < kInterpPerBin * nbins) return false;
+    const Workspace ws((size_t)bins_words(nbins, a.n) * sizeof(int), st);
+    if (!ws.p) return false;
+    launch_binning(PlaceKey<4>{a}, b, nbins, a.n, bin_one_max(4), (int *)ws.p, st);
+    hipLaunchKernelGGL(k_interp3d_bins<4>, dim3((unsigned)nbins), dim3(256), 0, st, a, b);
     return true;
 }
 
@@ -703,6 +845,15 @@ int smi_interpolate_3d(int order, const double *Ex, const double *Ey, const doub
     Dbl3 di{{1.0 / cell_length[0], 1.0 / cell_length[1], 1.0 / cell_length[2]}};
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid(nblk(n, 256)), block(256);
+    const Interp3Args a{{Ex, Ey, Ez, Bxm, Bym, Bzm}, NP, D, di, n, {x, y, z}, Epart, Bpart, iold, deltaold};
+    try {
+        if (launch_interp_bins(order, a, st)) {
+            OP_CHECK();
+            return SMI_OK;
+        }
+    } catch (const std::exception &e) {
+        return op_fail(SMI_ERR_HIP, e.what());
+    }
     const bool small = (int64_t)(np[0] + 1) * (np[1] + 1) * (np[2] + 1) < (1ll << 29);
 #define SMI_INTERP(O, T)                                                                                             \
     hipLaunchKernelGGL((k_interp3d<O, T>), grid, block, 0, st, Ex, Ey, Ez, Bxm, Bym, Bzm, NP, D, di, n, x, y, z, Epart, \
