@@ -192,9 +192,9 @@ __global__ void __launch_bounds__(128, 2) k_proj3d_atomic(Proj3Args a)
 // Binning pays from this many particles on.  Sorted / unsorted arrays,
 // microseconds, per-particle atomics against bins: order 2, 4,096 particles
 // 20 / 31 against 22 / 22, 8,192 29 / 47 against 23 / 23, 32,768 88 / 160
-// against 39 / 40, 2.1e6 4,000 / 7,222 against 211 / 473; order 4, 64
+// against 39 / 40, 2.1e6 4,000 / 7,222 against 180 / 481; order 4, 64
 // particles 39 / 40 against 24 / 23, 512 54 / 79 against 24 / 24, 32,768 432 /
-// 775 against 79 / 64, 2.1e6 19,020 / 34,860 against 907 / 666.
+// 775 against 61 / 62, 2.1e6 19,020 / 34,860 against 622 / 670.
 constexpr int64_t bin_min(int order) { return order == 2 ? 8192 : 64; }
 
 // Up to this many particles one workgroup does all of the binning: four
@@ -418,7 +418,11 @@ __device__ inline bool bin_deposit(const Proj3Args &a, int64_t i, double *sJ)
 
 // One workgroup per bin.  The particles that change node are queued and
 // deposited by a second pass, so that the first runs the narrow stencil with
-// all lanes.
+// all lanes.  A lane takes a run of the bin's list and a wavefront every fourth
+// place of its lanes' runs: neighbours in the list, mostly of one node where
+// the arrays are in cell order, do not meet on the same words (order 4, 2.1e6
+// particles in cell order 911 us with neighbours on neighbouring lanes, 622 so;
+// in no order 668 / 670).
 template <int ORDER>
 __global__ void __launch_bounds__(256) k_proj3d_bins(Proj3Args a, Bins b)
 {
@@ -432,8 +436,9 @@ __global__ void __launch_bounds__(256) k_proj3d_bins(Proj3Args a, Bins b)
     for (int t = threadIdx.x; t < 3 * BT::SC; t += blockDim.x) sJ[t] = 0.;
     if (threadIdx.x == 0) sQn = 0;
     __syncthreads();
-    for (int j = s + (int)threadIdx.x; j < e; j += blockDim.x) {
-        const int i = b.list[j];
+    const int n = e - s, per = (n + 63) / 64, first = (threadIdx.x & 63) * per;
+    for (int k = threadIdx.x >> 6; k < per && first + k < n; k += blockDim.x >> 6) {
+        const int i = b.list[s + first + k];
         if (bin_deposit<ORDER, false>(a, i, sJ)) continue;
         const int q = atomicAdd(&sQn, 1);
         if (q < QCAP) sQ[q] = i;
