@@ -223,7 +223,7 @@ void *smi_stream(smi_context *ctx);
  * clusters, so that neighbouring clusters share L2 lines; 0 = grid order. */
 #define SMI_TUNE_XCD 5
 /* SMI_TUNE_TILE (mixed form): LDS tile shape of the particle kernel, 1 = J
- * rows padded by one 64-bit word (fewer bank conflicts of the tile atomics
+ * rows and x-planes padded (fewer bank conflicts of the tile atomics
  * on dense plasmas), 0 = unpadded. */
 #define SMI_TUNE_TILE 6
 /* SMI_TUNE_TILE_X (mixed form, order 2): the patch tile one workgroup

@@ -1,8 +1,8 @@
 """Canonical order inside crowded cells, against the oracle's, bit for bit.
 
-The in-cell pass ranks up to 16 particles in a thread's registers, up to 32 by
-half a wavefront, up to 256 by a whole one with up to four places per lane,
-and the rest by a workgroup: every edge of these ranges appears as a cell's
+The in-cell pass ranks cells of up to 256 particles with one lane per particle,
+whole cells into batches of 512 places, and the rest by a workgroup: cells at
+and around powers of two and every edge of these ranges appears as a cell's
 number of particles, after one step in which a third of the particles change
 cell (the fields are zero, so positions are the oracle's in every mode), for
 several species of different sizes sorted in shared launches.
