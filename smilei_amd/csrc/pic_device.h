@@ -286,21 +286,37 @@ __device__ inline double rsqrt_cubic(double x)
     return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// Boris push by the two cross products, fused.  The last factor, 1/gamma of
-// the new momentum, is rounded as boris() rounds it, so without fields the two
-// agree bit for bit.
+// Boris push, fused: by the two cross products up to |t|^2 = 1/2, by the rotation
+// matrix above.  Errors against 128-bit values, units of 2^-53 |u|, rms over
+// random directions, boris() / cross products / fused matrix: |t| 0.1 1.47 /
+// 0.65 / 1.42, 0.7 1.56 / 1.34 / 1.46, 2 1.51 / 1.67 / 1.34, 50 1.38 / 1.69 /
+// 1.27.  The last factor, 1/gamma of the new momentum, is rounded as boris()
+// rounds it, so without fields the two agree bit for bit.
 __device__ inline void boris_fused(double qmh, double dt, const double *E, const double *B, double *u, double *dxp,
                                    double &invgf)
 {
     const double ux = fma(qmh, E[0], u[0]), uy = fma(qmh, E[1], u[1]), uz = fma(qmh, E[2], u[2]);
     const double f = qmh * rsqrt_cubic(fma(ux, ux, fma(uy, uy, fma(uz, uz, 1.))));
     const double tx = f * B[0], ty = f * B[1], tz = f * B[2];
-    const double s = 2. * rcp_cubic(fma(tx, tx, fma(ty, ty, fma(tz, tz, 1.))));
-    const double vx = fma(uy, tz, fma(-uz, ty, ux)), vy = fma(uz, tx, fma(-ux, tz, uy)),
-                 vz = fma(ux, ty, fma(-uy, tx, uz));
-    const double sx = s * tx, sy = s * ty, sz = s * tz;
-    const double ax = fma(qmh, E[0], fma(vy, sz, fma(-vz, sy, ux))), ay = fma(qmh, E[1], fma(vz, sx, fma(-vx, sz, uy))),
-                 az = fma(qmh, E[2], fma(vx, sy, fma(-vy, sx, uz)));
+    const double d = fma(tx, tx, fma(ty, ty, fma(tz, tz, 1.)));
+    const double s = 2. * rcp_cubic(d);
+    double ax, ay, az;
+    if (d <= 1.5) {
+        const double vx = fma(uy, tz, fma(-uz, ty, ux)), vy = fma(uz, tx, fma(-ux, tz, uy)),
+                     vz = fma(ux, ty, fma(-uy, tx, uz));
+        const double sx = s * tx, sy = s * ty, sz = s * tz;
+        ax = fma(vy, sz, fma(-vz, sy, ux));
+        ay = fma(vz, sx, fma(-vx, sz, uy));
+        az = fma(vx, sy, fma(-vy, sx, uz));
+    } else {
+        const double xx = tx * tx, yy = ty * ty, zz = tz * tz;
+        ax = s * fma(0.5 * (1. + xx - yy - zz), ux, fma(fma(tx, ty, tz), uy, fma(tz, tx, -ty) * uz));
+        ay = s * fma(fma(tx, ty, -tz), ux, fma(0.5 * (1. - xx + yy - zz), uy, fma(ty, tz, tx) * uz));
+        az = s * fma(fma(tz, tx, ty), ux, fma(fma(ty, tz, -tx), uy, 0.5 * (1. - xx - yy + zz) * uz));
+    }
+    ax = fma(qmh, E[0], ax);
+    ay = fma(qmh, E[1], ay);
+    az = fma(qmh, E[2], az);
     double gi = 1. / sqrt(1.0 + ax * ax + ay * ay + az * az);
     invgf = gi;
     u[0] = ax;
