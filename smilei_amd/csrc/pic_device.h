@@ -283,7 +283,7 @@ __device__ inline double rcp_cubic(double x)
 __device__ inline double rsqrt_cubic(double x)
 {
     const double y = __builtin_amdgcn_rsq(x), e = fma(-x * y, y, 1.);
-    return fma(y * e, fma(0.375, e, 0.5), y);
+    return e != e ? y : fma(y * e, fma(0.375, e, 0.5), y);  // x infinite: y = 0, and the product above NaN
 }
 
 // Boris push, fused: by the two cross products up to |t|^2 = 1/2, by the rotation
