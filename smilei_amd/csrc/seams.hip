@@ -81,30 +81,37 @@ __device__ inline int bin_coords(const SeamArgs &a, int b, int *bc)
     return b;
 }
 
-// Particle range of bin b, and this thread's share of it: a contiguous chunk
-// per thread with cell_sorting (neighbours in a cell land on one thread), a
-// strided walk otherwise (Projector3D2OrderGPUKernelCUDAHIP.cu:237-256 picks
-// the same two orders).  Only the order of the tile atomics differs.  The
-// chunks go to the lanes of different wavefronts in turn, so that the lanes of
-// one wavefront lie the bin's size / 64 apart, in different cells: with
-// neighbouring chunks on neighbouring lanes their atomics met on the same
-// words (currents of 16 particles per cell 44.5 us against 42.3).
-__device__ inline void bin_share(const SeamArgs &a, int b, int64_t &beg, int64_t &end, int64_t &stride)
+// Calls f(i) for this thread's particles of bin b: with cell_sorting runs of
+// neighbours (mostly of one cell) per thread, a strided walk otherwise
+// (Projector3D2OrderGPUKernelCUDAHIP.cu:237-256 picks such a pair of orders).
+// Only the order of the tile atomics differs.  The runs go to the lanes of
+// different wavefronts in turn, so that the lanes of one wavefront mostly lie in
+// different cells: with neighbouring runs on neighbouring lanes their atomics met
+// on the same words (currents of 16 particles per cell 44.5 us against 42.3).
+// A run is four particles at most, 1,024 of the bin at a time, where there are
+// more bins than the caches hold the lines of: each thread of a run reads 8 bytes
+// of its own line of 13 arrays.  Both seams, 64 particles per cell, few movers
+// / many: 512 bins 656 / 666 us with one run a thread, 305 / 420 with runs of
+// four; 4,096 bins 4,887 / 4,944 and 2,372 / 2,977; but 64 bins 179 / 214 and 192
+// / 249, 128 bins (of 128 per cell) 372 / 421 and 369 / 523, 256 690 / 699 and
+// 372 / 528.
+constexpr int kSeamThreads = 256, kSeamRun = 4, kSeamFewBins = 128;
+
+template <class F>
+__device__ inline void for_bin(const SeamArgs &a, int b, F f)
 {
     int64_t first = b == 0 ? 0 : a.bin_index[b - 1], last = a.bin_index[b];
     first = first < 0 ? 0 : (first > a.n ? a.n : first);
     last = last < first ? first : (last > a.n ? a.n : last);
-    if (a.cell_sorting) {
-        const int64_t per = (last - first + blockDim.x - 1) / blockDim.x;
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        beg = first + (int64_t)(lane * (blockDim.x >> 6) + wave) * per;
-        beg = beg < last ? beg : last;
-        end = beg + per < last ? beg + per : last;
-        stride = 1;
-    } else {
-        beg = first + threadIdx.x;
-        end = last;
-        stride = blockDim.x;
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int64_t once = !a.cell_sorting ? kSeamThreads
+                                         : (gridDim.x <= kSeamFewBins ? last - first : kSeamRun * kSeamThreads);
+    const int place = a.cell_sorting ? lane * (kSeamThreads / 64) + wave : threadIdx.x;
+    for (int64_t i0 = first; i0 < last; i0 += once) {
+        const int64_t end = i0 + once < last ? i0 + once : last;
+        const int per = (int)((end - i0 + kSeamThreads - 1) / kSeamThreads);
+        const int64_t mine = i0 + (int64_t)place * per;
+        for (int64_t i = mine; i < mine + per && i < end; ++i) f(i);
     }
 }
 
@@ -152,7 +159,7 @@ __device__ inline void seam_deposit(const SeamArgs &a, int64_t i, const int *o, 
 // its node adds 54 points (300 walked with a test for zero before: 84 us for
 // 524,288 particles in 512 bins, 42 now); the others are queued and
 // deposited by a second pass, so that the lanes of the first agree.
-__global__ void __launch_bounds__(256) k_seam_currents(SeamArgs a)
+__global__ void __launch_bounds__(kSeamThreads) k_seam_currents(SeamArgs a)
 {
     constexpr int QCAP = 256;
     __shared__ double sJ[3 * kCC];
@@ -164,23 +171,21 @@ __global__ void __launch_bounds__(256) k_seam_currents(SeamArgs a)
     for (int t = threadIdx.x; t < 3 * kCC; t += blockDim.x) sJ[t] = 0.;
     if (threadIdx.x == 0) sQn = 0;
     __syncthreads();
-    int64_t beg, end, stride;
-    bin_share(a, b, beg, end, stride);
-    for (int64_t i = beg; i < end; i += stride) {
+    for_bin(a, b, [&](int64_t i) {
         int o[3], node[3], sh[3];
         double pn[3];
         if (!seam_particle(a, i, bc, o, node, sh, pn)) {
             atomicOr(a.err, 1);
-            continue;
+            return;
         }
         if ((sh[0] | sh[1] | sh[2]) == 0) {
             seam_deposit<false>(a, i, o, node, pn, sJ);
-            continue;
+            return;
         }
         const int q = atomicAdd(&sQn, 1);
         if (q < QCAP) sQ[q] = i;
         else seam_deposit<true>(a, i, o, node, pn, sJ);
-    }
+    });
     __syncthreads();
     const int nq = sQn < QCAP ? sQn : QCAP;
     for (int q = threadIdx.x; q < nq; q += blockDim.x) {
@@ -211,7 +216,7 @@ __global__ void __launch_bounds__(256) k_seam_currents(SeamArgs a)
     }
 }
 
-__global__ void __launch_bounds__(256) k_seam_density(SeamArgs a)
+__global__ void __launch_bounds__(kSeamThreads) k_seam_density(SeamArgs a)
 {
     __shared__ double sR[kCC];
     const int b = blockIdx.x;
@@ -219,14 +224,12 @@ __global__ void __launch_bounds__(256) k_seam_density(SeamArgs a)
     bin_coords(a, b, bc);
     for (int t = threadIdx.x; t < kCC; t += blockDim.x) sR[t] = 0.;
     __syncthreads();
-    int64_t beg, end, stride;
-    bin_share(a, b, beg, end, stride);
-    for (int64_t i = beg; i < end; i += stride) {
+    for_bin(a, b, [&](int64_t i) {
         int o[3], node[3], sh[3];
         double pn[3], S1[3][3];
         if (!seam_particle(a, i, bc, o, node, sh, pn)) {
             atomicOr(a.err, 1);
-            continue;
+            return;
         }
         // S1: the new position's weights on the 5-point window of the old
         // node (init_S1, Projector3D2OrderGPUKernelCUDAHIP.cu:116-131), whose
@@ -246,7 +249,7 @@ __global__ void __launch_bounds__(256) k_seam_density(SeamArgs a)
 #pragma unroll
                 for (int k = 0; k < 3; ++k) atomicAdd(&r[u * kCX + v * kCY + k], t * S1[2][k]);
             }
-    }
+    });
     __syncthreads();
     for (int t = threadIdx.x; t < kCT3; t += blockDim.x) {
         const int u = t / (kCT * kCT), v = (t / kCT) % kCT, k = t % kCT;
