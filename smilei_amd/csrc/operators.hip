@@ -215,21 +215,19 @@ struct Bins {
     int nbins, share;
     int *count;     // per bin
     int *start;     // per bin, and the total
-    int *further;   // per bin, the further shares of the bins before it; and the total
     int *key, *rank, *list;  // per particle
+    int2 *further;  // bin and number of the further shares of crowded bins
+    int *nfurther;
 };
 
 // A crowded bin is worked on in equal shares of at most b.share particles, by
 // as many workgroups: with one workgroup per bin a species that lies in a few
 // bins was left to a few CUs (6e5 particles within 2^3 cells, order 4:
 // interpolation 34 ms, projection 66 ms; 0.14 and 0.43 ms in shares).
-__device__ inline int bin_shares(const Bins &b, int count)
-{
-    return count > b.share ? (count + b.share - 1) / b.share : 1;
-}
+__device__ inline int bin_shares(const Bins &b, int count) { return (count + b.share - 1) / b.share; }
 
-// Work items: the first share of every bin, then the further ones, in the
-// order of the bins; empty beyond them.
+// Work items: the first share of every bin, then the further ones; empty
+// beyond them.
 struct Share {
     int bin, first, last;  // its places in the list
 };
@@ -237,52 +235,76 @@ __device__ inline Share bin_item(const Bins &b, int item)
 {
     int bin = item, k = 0;
     if (item >= b.nbins) {
-        const int h = item - b.nbins;
-        if (h >= b.further[b.nbins]) return Share{0, 0, 0};
-        int lo = 0, hi = b.nbins;  // the last bin with no more than h further shares before it
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (b.further[mid] <= h) lo = mid;
-            else hi = mid;
-        }
-        bin = lo;
-        k = 1 + h - b.further[lo];
+        if (item - b.nbins >= *b.nfurther) return Share{0, 0, 0};
+        const int2 f = b.further[item - b.nbins];
+        bin = f.x;
+        k = f.y;
     }
     Share w{bin, b.start[bin], b.start[bin + 1]};
-    const int shares = bin_shares(b, w.last - w.first);
-    if (shares > 1) {
-        const int per = (w.last - w.first + shares - 1) / shares;
+    const int count = w.last - w.first;
+    if (count > b.share) {
+        const int shares = bin_shares(b, count), per = (count + shares - 1) / shares;
         w.first += k * per;
         w.last = w.last - w.first < per ? w.last : w.first + per;
     }
     return w;
 }
 
-// Sum over the threads of a 1024-thread workgroup before this one, and the
-// total: particles in the low word, further shares in the high one.
-__device__ inline uint64_t bin_prefix(uint64_t sum, uint64_t *part, uint64_t &total)
+// Starts of all bins from their counts, and the further shares, by one
+// workgroup, 4,096 bins at a time; keep: the starts take the counts' place too.
+constexpr int kBinThreads = 1024;
+__device__ inline void bin_scan(const Bins &b, int *count, bool keep)
 {
+    constexpr int WAVES = kBinThreads / 64;
+    __shared__ int part[2][WAVES];
+    __shared__ int nfurther;
+    if (threadIdx.x == 0) nfurther = 0;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint64_t incl = sum;
+    int before = 0;
+    for (int q0 = 0, k = 0; q0 < b.nbins; q0 += 4 * kBinThreads, k ^= 1) {
+        const int q = q0 + 4 * threadIdx.x, m = b.nbins - q;
+        int c[4] = {0, 0, 0, 0};
+        if (m >= 4) {
+            const int4 v = *reinterpret_cast<const int4 *>(count + q);
+            c[0] = v.x;
+            c[1] = v.y;
+            c[2] = v.z;
+            c[3] = v.w;
+        } else {
+            for (int i = 0; i < m; ++i) c[i] = count[q + i];
+        }
+        const int sum = c[0] + c[1] + c[2] + c[3];
+        int incl = sum;
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint64_t t = __shfl_up((unsigned long long)incl, o, 64);
-        if (lane >= o) incl += t;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += t;
+        }
+        if (lane == 63) part[k][wave] = incl;
+        __syncthreads();
+        int at = before + incl - sum;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            if (w < wave) at += part[k][w];
+            before += part[k][w];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (i >= m) break;
+            b.start[q + i] = at;
+            if (keep) count[q + i] = at;
+            at += c[i];
+            if (c[i] > b.share) {
+                const int more = bin_shares(b, c[i]) - 1, f = atomicAdd(&nfurther, more);
+                for (int j = 0; j < more; ++j) b.further[f + j] = make_int2(q + i, j + 1);
+            }
+        }
     }
-    if (lane == 63) part[wave] = incl;
     __syncthreads();
-    uint64_t at = incl - sum;
-    total = 0;
-#pragma unroll
-    for (int w = 0; w < 16; ++w) {
-        if (w < wave) at += part[w];
-        total += part[w];
+    if (threadIdx.x == 0) {
+        b.start[b.nbins] = before;
+        *b.nfurther = nfurther;
     }
-    return at;
-}
-__device__ inline uint64_t bin_weight(const Bins &b, int count)
-{
-    return (uint64_t)(uint32_t)count | (uint64_t)(bin_shares(b, count) - 1) << 32;
 }
 
 // Bin of particle i by its old node, or -1 for one whose stencil would leave
@@ -334,7 +356,7 @@ __global__ void __launch_bounds__(256) k_bin_count(Key of, Bins b)
 // queue up otherwise (order 2, whole call, with k_bin_count: 2.6e5 particles
 // 88 us in cell order and 131 shuffled, here 56 and 69; 2.1e6 307 and 558, here
 // 211 and 473).
-constexpr int kBinLds = 8192, kBinThreads = 1024;
+constexpr int kBinLds = 8192;
 
 template <class Key>
 __device__ inline void bin_count_lds(const Key &of, const Bins &b, int nbins, int64_t i0, int per, int *h)
@@ -381,24 +403,9 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_count_lds(Key of, Bins b, i
 template <class Key>
 __global__ void __launch_bounds__(kBinThreads) k_bin_one(Key of, Bins b, int nbins, int per)
 {
-    __shared__ int h[kBinLds];
-    __shared__ uint64_t part[kBinThreads / 64];
+    __shared__ __align__(16) int h[kBinLds];
     bin_count_lds(of, b, nbins, 0, per, h);
-    const int run = (nbins + kBinThreads - 1) / kBinThreads;
-    const int q0 = threadIdx.x * run, q1 = q0 + run < nbins ? q0 + run : nbins;
-    uint64_t sum = 0;
-    for (int q = q0; q < q1; ++q) sum += bin_weight(b, h[q]);
-    uint64_t total, at = bin_prefix(sum, part, total);
-    for (int q = q0; q < q1; ++q) {
-        const int c = h[q];
-        b.start[q] = h[q] = (int)(uint32_t)at;
-        b.further[q] = (int)(at >> 32);
-        at += bin_weight(b, c);
-    }
-    if (threadIdx.x == 0) {
-        b.start[nbins] = (int)(uint32_t)total;
-        b.further[nbins] = (int)(total >> 32);
-    }
+    bin_scan(b, h, true);
     __syncthreads();
 #pragma unroll 4
     for (int k = 0; k < per; ++k) {
@@ -407,37 +414,9 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_one(Key of, Bins b, int nbi
     }
 }
 
-// Start of every bin, by one workgroup, 4,096 bins at a time.
-__global__ void __launch_bounds__(1024) k_bin_scan(Bins b)
+__global__ void __launch_bounds__(kBinThreads) k_bin_scan(Bins b)
 {
-    __shared__ uint64_t part[2][16];
-    uint64_t before = 0;
-    for (int q0 = 0, k = 0; q0 < b.nbins; q0 += 4096, k ^= 1) {
-        const int q = q0 + 4 * threadIdx.x, m = b.nbins - q;
-        int4 c{0, 0, 0, 0};
-        if (m >= 4) {
-            c = *reinterpret_cast<const int4 *>(b.count + q);
-        } else {
-            if (m > 0) c.x = b.count[q];
-            if (m > 1) c.y = b.count[q + 1];
-            if (m > 2) c.z = b.count[q + 2];
-        }
-        const uint64_t w[4] = {bin_weight(b, c.x), bin_weight(b, c.y), bin_weight(b, c.z), bin_weight(b, c.w)};
-        uint64_t total, at = before + bin_prefix(w[0] + w[1] + w[2] + w[3], part[k], total);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (i < m) {
-                b.start[q + i] = (int)(uint32_t)at;
-                b.further[q + i] = (int)(at >> 32);
-            }
-            at += w[i];
-        }
-        before += total;
-    }
-    if (threadIdx.x == 0) {
-        b.start[b.nbins] = (int)(uint32_t)before;
-        b.further[b.nbins] = (int)(before >> 32);
-    }
+    bin_scan(b, b.count, false);
 }
 
 __global__ void __launch_bounds__(256) k_bin_fill(Bins b, int64_t n)
@@ -720,10 +699,6 @@ int op_fail(int code, const std::string &m)
     return code;
 }
 
-// The binned projection where it is the faster one and has its scratch;
-// false otherwise.
-int64_t bins_words(int64_t nbins, int64_t n) { return 3 * nbins + 2 + 3 * n; }
-
 // Particles of a share: 1,024, more where a uniform plasma has more to a bin
 // (a bin with four times the mean is split) as long as there are 2,048 shares.
 // Uniform, 8.4e6 particles and 1,223 to a bin, order 4: interpolation 1,372 us
@@ -736,16 +711,20 @@ int64_t share_size(int64_t nbins, int64_t n) { return std::max<int64_t>(1024, st
 // took 432 us instead of 407).
 int64_t share_blocks(int64_t nbins, int64_t n) { return nbins + n / share_size(nbins, n); }
 
+// 4-byte words of scratch of the binning.
+int64_t bins_words(int64_t nbins, int64_t n) { return 2 * (n / share_size(nbins, n)) + 2 + 2 * nbins + 2 + 3 * n; }
+
 // Lists the n particles by bin: b.start and b.list, in ws (bins_words).
 template <class Key>
 void launch_binning(const Key &of, Bins &b, int64_t nbins, int64_t n, int64_t one_max, int *ws, hipStream_t st)
 {
-    b.count = ws;
     b.nbins = (int)nbins;
     b.share = (int)share_size(nbins, n);
-    b.start = b.count + nbins;
-    b.further = b.start + nbins + 1;
-    b.key = b.further + nbins + 1;
+    b.count = ws;  // (read four at a time)
+    b.further = (int2 *)(b.count + (nbins + 1) / 2 * 2);
+    b.nfurther = (int *)(b.further + n / b.share);
+    b.start = b.nfurther + 2;
+    b.key = b.start + nbins + 1;
     b.rank = b.key + n;
     b.list = b.rank + n;
     const dim3 wide(kBinThreads);
@@ -764,10 +743,12 @@ void launch_binning(const Key &of, Bins &b, int64_t nbins, int64_t n, int64_t on
     } else {
         hipLaunchKernelGGL(k_bin_count<Key>, dim3(nblk(n, 256)), dim3(256), 0, st, of, b);
     }
-    hipLaunchKernelGGL(k_bin_scan, dim3(1), dim3(1024), 0, st, b);
+    hipLaunchKernelGGL(k_bin_scan, dim3(1), wide, 0, st, b);
     hipLaunchKernelGGL(k_bin_fill, dim3(nblk(n, 256)), dim3(256), 0, st, b, n);
 }
 
+// The binned projection where it is the faster one and has its scratch;
+// false otherwise.
 bool launch_bins(int order, const Proj3Args &a, hipStream_t st)
 {
     if (a.n < bin_min(order) || a.n >= (1ll << 31)) return false;
