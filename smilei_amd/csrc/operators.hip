@@ -758,7 +758,14 @@ bool launch_bins(int order, const Proj3Args &a, hipStream_t st)
         b.nb[d] = (a.dims[(d + 1) % 3][d] + 3) / 4;
         nbins *= b.nb[d];
     }
-    if (nbins > a.n) return false;  // less than one particle per bin
+    // Sparse: a workgroup per bin for one particle, and at order 2 the launches of
+    // the binning, which cost what the atomics of 5,000 particles do.  Order 2,
+    // atomics against bins, cell order: 4,913 bins, 8,192 particles 37.5 / 35.2 us,
+    // 10,000 42.3 / 38.2; 8,000 bins, 10,000 42.6 / 47.9, 14,000 55.1 / 56.5, 16,384
+    // 62.8 / 56.7; 9,261 bins, 16,384 65.0 / 54.1; 15,625 bins, 22,000 82.7 / 72.8;
+    // 17,576 bins, 18,000 70 / 78, 24,000 89.6 / 78.6; 35,937 bins, 42,500 158 /
+    // 133; 274,625 bins, 280,000 1,007 / 1,004.  Order 4, 6,859 bins, 7,000 139 / 67.
+    if (a.n < (order == 2 ? nbins + std::min<int64_t>(2 * nbins / 3, 5120) : nbins)) return false;
     if (share_blocks(nbins, a.n) >= (1ll << 24)) return false;  // 2^32 threads a launch
     const Workspace ws((size_t)bins_words(nbins, a.n) * sizeof(int), st);
     if (!ws.p) return false;

@@ -1,0 +1,45 @@
+"""smi_currents_3d with about one particle per bin, order 2: the 10,000
+particles take no longer in a patch of 8,000 or 9,261 bins than in one of 10,648,
+where they are too few to be binned (binned at 1.25 particles to a bin 1.9 times
+as long).  Small patches of few particles still agree with index order
+(fewer than 2,000 contributions to a point: 1e-12 of the largest |J|).
+"""
+import time
+
+import pytest
+
+from tests.test_gpu_binned_currents import arrays, call, inputs
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def per_call(n):
+    begin, dev, pos = inputs(2, n, 10000, "cell order", 3)
+    J = arrays(2, n)
+    best = 1e9
+    for _ in range(8):
+        torch.cuda.synchronize()
+        t = time.perf_counter()
+        for _ in range(200):
+            call(2, n, begin, dev, pos, 0, J)
+        torch.cuda.synchronize()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+@pytest.mark.parametrize("n", [(75, 75, 75), (77, 77, 77)])
+def test_few_particles_to_a_bin_cost_no_more(n):
+    assert per_call(n) <= 1.07 * per_call((83, 83, 83))
+
+
+@pytest.mark.parametrize("n,m", [((75, 75, 75), 11999), ((75, 75, 75), 12000), ((60, 76, 72), 9000)])
+def test_both_sides_of_the_line(n, m):
+    begin, dev, pos = inputs(2, n, m, "any", 9)
+    want, got = arrays(2, n), arrays(2, n)
+    call(2, n, begin, dev, pos, 1, want)
+    call(2, n, begin, dev, pos, 0, got)
+    torch.cuda.synchronize()
+    for a, b in zip(want, got):
+        assert float((a - b).abs().max()) <= 1e-12 * float(a.abs().max())
