@@ -616,7 +616,7 @@ int smi_add_species(smi_context *c, const char *name, double mass, double charge
     s.sb.perm = dalloc<int32_t>(capacity);
     s.sb.tmp = dalloc<int32_t>(capacity);
     s.sb.big = dalloc<int32_t>(capacity / 17 + 1);
-    s.sb.nbig = dalloc<int32_t>(2);
+    s.sb.nbig = dalloc<int32_t>(3);
     if (c->p.deposit != SMI_DEPOSIT_DETERMINISTIC) s.sb.rank = dalloc<int32_t>(capacity);
     s.sb.nbsum = sort_bsum_size(c->g.ncells);
     s.sb.bsum = dalloc<int32_t>(s.sb.nbsum);

@@ -171,8 +171,9 @@ struct SortBufs {
     int32_t *perm;     // cap
     int32_t *tmp;      // cap (cell-major order before the interleaved layout)
     int32_t *rank;     // cap (tie-break of the canonical order of the particles that left their cluster)
-    int32_t *big;      // cap / 17 + 1, or null: cells of more than 256 particles, which a workgroup sorts
-    int32_t *nbig;     // 2 (count, queue head of `big`)
+    int32_t *big;      // cap / 17 + 1: cells of more than 256 and of more than 64 particles, which a workgroup / a
+                       // wavefront sorts (null: no order inside cells)
+    int32_t *nbig;     // 3 (count and queue head of the former, count of the latter)
     int32_t *bsum;     // scan scratch
     int64_t nbsum;
     // Placed stayers: when the particle kernel is given `stay`, a particle

@@ -695,7 +695,7 @@ int64_t align_words(int64_t w) { return (w + kAlignWords - 1) / kAlignWords * kA
 int64_t smi::seams::sort_scratch_words(const Geom &g, int64_t n, int nstage)
 {
     const int64_t nc = g.ncells, m = n > 0 ? n : 1;
-    return align_words(nc) + align_words(nc + 1) + 2 * align_words(m) + align_words(m / 17 + 1) + align_words(2) +
+    return align_words(nc) + align_words(nc + 1) + 2 * align_words(m) + align_words(m / 17 + 1) + align_words(3) +
            align_words(sort_bsum_size(nc)) + align_words((nc + 3) / 4) + align_words(nc / g.cells_per_cl) +
            align_words(m) + nstage * align_words(2 * m) + align_words(1);
 }
@@ -722,7 +722,7 @@ SortScratch smi::seams::carve_sort_scratch(const Geom &g, int64_t n, int32_t *ba
     s.sb.perm = take(m);
     s.sb.tmp = take(m);
     s.sb.big = take(m / 17 + 1);
-    s.sb.nbig = take(2);
+    s.sb.nbig = take(3);
     s.sb.nbsum = sort_bsum_size(nc);
     s.sb.bsum = take(s.sb.nbsum);
     s.sb.stay = (uint8_t *)take((nc + 3) / 4);

@@ -7,13 +7,15 @@
 // with one device-wide counting sort by destination cell, since the push
 // kernel already computed every particle's destination patch and cell:
 //   1. histogram of destination cells          (int32 atomics)
-//   2. exclusive scan -> cell_off               (3-phase block scan)
+//   2. exclusive scan -> cell_off               (block scan in one to three launches)
 //   3. scatter of slot indices into buckets     (atomic count-down, which
 //      also returns the histogram to zero for the next step)
 //   4. per-bucket rank sort by (direction of motion, source slot), the
 //      canonical order of particles inside a cell.
 // The particle data itself is not moved here: the next step's particle
 // kernel reads its input through `perm`.
+#include <algorithm>
+
 #include "kernels.h"
 #include "pic_device.h"
 
@@ -142,7 +144,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_apply(SortSet set, int64_
     const int32_t *__restrict__ bsum = S.bsum;
     uint8_t *__restrict__ stay = S.stay;
     int32_t *__restrict__ clus_old = S.clus_old;
-    if (S.nbig && blockIdx.x == 0 && threadIdx.x < 2) S.nbig[threadIdx.x] = 0;
+    if (S.nbig && blockIdx.x == 0 && threadIdx.x < 3) S.nbig[threadIdx.x] = 0;
     int before = 0;
     if (pref == kPrefScanned) {
         before = bsum[blockIdx.x];
@@ -308,10 +310,12 @@ __global__ void __launch_bounds__(kScatThreads) k_scatter(SortSet set, int cpc, 
 // pairs are distinct because slots are.  What bounds it is the chain place ->
 // slot -> key of loads from memory, hence the places in flight, eight
 // wavefronts per SIMD (64 registers, one of them spilled; at seven 72 against
-// 54 us) and the 18 KB of LDS.  Cells of more than kFixMid particles go to
-// the work list `big` (count in nbig[0]) for k_bucket_fix_big, or, without a
-// list, to an insertion sort in memory.  The stores of a batch follow the loads
-// of all its places, so the in-place case (dst == src) is safe.
+// 54 us) and the 18 KB of LDS.  Cells of more than `most` particles (fix_most) go
+// to the work lists of k_bucket_fix_big: a wavefront with many of them would
+// work on them for long after the rest of the chip is done (16^3 cells of 130
+// particles in a grid of 64^3, two species: 1,055 us a sort with cells of up to
+// 256 ranked here, 140 so; of 300, 960 and 285).  The stores of a batch follow
+// the loads of all its places, so the in-place case (dst == src) is safe.
 // 2D plasma, 2 x 2.6e5 cells of 16 particles: 54 us; 118 us with a thread per
 // cell of up to 16 particles and half a wavefront per cell of up to 32.
 // 3D, 2.6e5 cells of 8: 69 -> 29 us; 2 x 4.2e6 cells of 8: 453 -> 378 us.
@@ -319,11 +323,10 @@ __global__ void __launch_bounds__(kScatThreads) k_scatter(SortSet set, int cpc, 
 // cpc > 0: every particle is written to its lane-interleaved slot of the
 // cluster in dst.  The tie-break value of source slot v is tie[v] when tie
 // is given, else v.
-constexpr int kFixMid = 256;
+constexpr int kFixMid = 64;
 constexpr int kFixPer = 8;
-constexpr int kFixBatch = 64 * kFixPer;  // at least kFixMid: a batch holds one cell at least
+constexpr int kFixBatch = 64 * kFixPer;  // at least kFixWave: a batch holds one cell at least
 constexpr int kFixAhead = 4;             // keys read per step of the ranking
-static_assert(kFixBatch >= kFixMid, "a batch holds whole cells");
 
 // Where the tie-breaks come from: tie[v] (the cell-major position of slot
 // v in the previous sorted order, recorded by the particle kernel), or v
@@ -392,6 +395,12 @@ __device__ inline int wave_append(bool want, int32_t *counter)
     return base + __popcll(m & ((1ull << lane) - 1));
 }
 
+// The lists of crowded cells: more than kFixWave particles in S.big (at most n /
+// 257 cells), up to kFixWave behind them (at most n / 65).
+constexpr int kFixWave = 256;
+static_assert(kFixBatch >= kFixWave, "a batch holds whole cells");
+__device__ inline int32_t *mid_list(const SortOne &S) { return S.big + S.n / (kFixWave + 1) + 1; }
+
 // Orders a wavefront's accesses to LDS that only it uses.
 __device__ inline void lds_order()
 {
@@ -410,7 +419,20 @@ inline int fix_cells(int64_t cells)
     return cells >= 64 * kFixWaves ? 64 : cells >= 32 * kFixWaves ? 32 : 16;
 }
 
-__global__ void __launch_bounds__(256, 8) k_bucket_fix(SortSet set, int64_t ncells, int wcells, int cpc, int lay, TieGeom G)
+// Largest cell that a wavefront of k_bucket_fix ranks (its `most`): 64, or where
+// the mean cell is crowded itself twice the mean, as long as there are enough
+// wavefronts for all cells to be ranked at once.  Uniform plasmas of 2 species, cells
+// ranked there / listed, us: 8,192 wavefronts (64^3 cells), 64 particles per
+// cell 980 / 1,249, 128 2,607 / 3,065, 200 5,119 / 4,698; 4,096 (32^3) 80 221 / 251,
+// 100 301 / 289; 2,048 (128^2) 64 114 / 131, 80 150 / 126; 512 (16^3) 56 87 / 89, 64
+// 106 / 94: the line lies at 48 particles and one more per 75 wavefronts.
+inline int fix_most(int64_t n, int64_t ncells, int64_t waves)
+{
+    const int64_t mean = n / ncells;
+    return (int)std::min<int64_t>(mean > 48 + waves / 75 ? kFixMid : std::max<int64_t>(2 * mean, kFixMid), kFixWave);
+}
+
+__global__ void __launch_bounds__(256, 8) k_bucket_fix(SortSet set, int64_t ncells, int wcells, int most, int cpc, int lay, TieGeom G)
 {
     const SortOne &S = set.s[blockIdx.y];
     const uint32_t *__restrict__ keys = S.keys;
@@ -436,29 +458,15 @@ __global__ void __launch_bounds__(256, 8) k_bucket_fix(SortSet set, int64_t ncel
         }
         T.range(g, ocs, ocn);
     }
-    if (S.big) {
-        const int ib = wave_append(n > kFixMid, &S.nbig[0]);
-        if (n > kFixMid) S.big[ib] = (int32_t)g;
-    } else if (n > kFixMid) {
-        for (int i = a + 1; i < a + n; ++i) {
-            const int32_t v = src[i];
-            const uint64_t kv = fix_key(keys, T, v, ocs, ocn);
-            int j = i - 1;
-            while (j >= a) {
-                const int32_t u = src[j];
-                const uint64_t ku = fix_key(keys, T, u, ocs, ocn);
-                if (ku <= kv) break;
-                src[j + 1] = u;
-                --j;
-            }
-            src[j + 1] = v;
-        }
-        if (cpc)
-            for (int i = a; i < a + n; ++i) dst[cs + layout_slot(lay, i - cs, cn)] = src[i];
+    if (__ballot(n > most)) {
+        const int iw = wave_append(n > most && n <= kFixWave, &S.nbig[2]);
+        if (n > most && n <= kFixWave) mid_list(S)[iw] = (int32_t)g;
+        const int ib = wave_append(n > kFixWave, &S.nbig[0]);
+        if (n > kFixWave) S.big[ib] = (int32_t)g;
     }
     // places of the lane's cell in the wavefront's run (in place, a single
     // particle is where it belongs), and where they begin
-    const int m = n > kFixMid || (n == 1 && !cpc) ? 0 : n;
+    const int m = n > most || (n == 1 && !cpc) ? 0 : n;
     int end = m;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -517,27 +525,57 @@ __global__ void __launch_bounds__(256, 8) k_bucket_fix(SortSet set, int64_t ncel
     }
 }
 
-// The cells of the work list (more than kFixMid particles; their number in
-// nbig[0], nbig[1] = 0 on entry), one workgroup per cell pulled from the
-// list until it is exhausted.  Up to kBigLds particles: bitonic sort of the
-// (key, slot) pairs in LDS.  More: each particle's rank = the number of
-// smaller keys, counted over the cell in LDS-staged chunks, kBigLds target
-// particles at a time (in place, cpc == 0, the cell is first copied to scr
-// so that no write can overtake a read).  Every workgroup exits once the
-// list is exhausted.
+// The cells of the work lists.  Up to kFixWave particles (nbig[2] cells): a
+// wavefront each, four places a lane, a place's rank counted over the cell's keys
+// in LDS, which all lanes read at the same time.  More (nbig[0] cells, nbig[1] =
+// 0 on entry): one workgroup per cell pulled from the list until it is
+// exhausted.  Up to kBigLds particles: bitonic sort of the (key, slot) pairs in
+// LDS.  More: each particle's rank = the number of smaller keys, counted over the
+// cell in LDS-staged chunks, kBigLds target particles at a time (in place, cpc ==
+// 0, the cell is first copied to scr so that no write can overtake a read).
+// Every workgroup exits once the lists are exhausted.
 constexpr int kBigThreads = 256;
 constexpr int kBigLds = 4096;
 constexpr int kBigPer = kBigLds / kBigThreads;
 constexpr int kBigBlocks = 1024;
 
-// Workgroups for the crowded cells of n particles: there are at most n / 257
-// such cells and usually none, and a workgroup that finds the list empty still
-// costs its dispatch (1,024 of them, with 48 KB of LDS each: 13 us per
-// species).  All 1,024 only where the mean cell is half way to crowded.
-inline unsigned big_blocks(int64_t n, int64_t ncells)
+// Workgroups for the crowded cells of n particles, of which there are usually
+// none: a workgroup that finds the lists empty ends at its first load
+// (1,024 of them cost no more than 192 that each asked the list for work: 4.2e6
+// particles 84.3 / 83.8 us a sort).
+inline unsigned big_blocks(int64_t n)
 {
-    const int64_t b = (n + 2047) / 2048, most = n > ncells * (kFixMid / 2) ? kBigBlocks : 192;
-    return (unsigned)(b < most ? b : most);
+    const int64_t b = (n + 2047) / 2048;
+    return (unsigned)(b < kBigBlocks ? b : kBigBlocks);
+}
+
+// Order of the cell of n <= 64 * PER particles from place a on, by one wavefront;
+// put(place, slot) stores; sk: 64 * PER keys of LDS.
+template <int PER, class Key, class Put>
+__device__ inline void rank_by_wave(const int32_t *src, int a, int n, uint64_t *sk, Key key, Put put)
+{
+    const int lane = threadIdx.x & 63;
+    int32_t v[PER];
+    uint64_t k[PER];
+    int r[PER];
+#pragma unroll
+    for (int q = 0; q < PER; ++q) v[q] = 64 * q + lane < n ? src[a + 64 * q + lane] : 0;
+#pragma unroll
+    for (int q = 0; q < PER; ++q) {
+        k[q] = 64 * q + lane < n ? key(v[q]) : ~0ull;
+        r[q] = 0;
+        sk[64 * q + lane] = k[q];
+    }
+    lds_order();
+    for (int j = 0; j < n; j += 2) {  // (an entry after the last is the largest key)
+        const uint64_t k0 = sk[j], k1 = sk[j + 1];
+#pragma unroll
+        for (int q = 0; q < PER; ++q) r[q] += (k0 < k[q] ? 1 : 0) + (k1 < k[q] ? 1 : 0);
+    }
+    lds_order();
+#pragma unroll
+    for (int q = 0; q < PER; ++q)
+        if (64 * q + lane < n) put(a + r[q], v[q]);
 }
 
 __global__ void __launch_bounds__(kBigThreads) k_bucket_fix_big(SortSet set, int cpc, int lay, TieGeom G)
@@ -552,8 +590,27 @@ __global__ void __launch_bounds__(kBigThreads) k_bucket_fix_big(SortSet set, int
     __shared__ uint64_t sK[kBigLds];
     __shared__ int32_t sV[kBigLds];
     __shared__ int sItem;
-    const int nb = nbig[0];
+    const int nb = nbig[0], nm = nbig[2];
+    if ((nb | nm) == 0) return;
     const int tid = threadIdx.x;
+    const int32_t *mid = mid_list(S);
+    for (int item = blockIdx.x * (kBigThreads / 64) + (tid >> 6); item < nm; item += gridDim.x * (kBigThreads / 64)) {
+        const int g = mid[item], a = cell_off[g];
+        int cs = 0, cn = 0, ocs, ocn;
+        if (cpc) {
+            const int cb = g & ~(cpc - 1);
+            cs = cell_off[cb];
+            cn = cell_off[cb + cpc] - cs;
+        }
+        T.range(g, ocs, ocn);
+        const int n = cell_off[g + 1] - a;
+        uint64_t *sk = sK + (tid >> 6) * kFixWave;
+        auto key = [&](int32_t v) { return fix_key(keys, T, v, ocs, ocn); };
+        auto put = [&](int pos, int32_t v) { dst[cpc ? cs + layout_slot(lay, pos - cs, cn) : pos] = v; };
+        if (n <= 128) rank_by_wave<2>(src, a, n, sk, key, put);
+        else rank_by_wave<4>(src, a, n, sk, key, put);
+    }
+    if (nb == 0) return;
     for (;;) {
         __syncthreads();  // the previous cell is done with the LDS arrays
         if (tid == 0) sItem = atomicAdd(&nbig[1], 1);
@@ -684,7 +741,6 @@ void launch_sort(const Geom &g, const SortTask *tasks, int ns, hipStream_t st, b
     const int cpc = layout ? g.cells_per_cl : 0;
     SortSet set{};
     int64_t most = 0;
-    bool big = false;
     for (int q = 0; q < ns; ++q) {
         const SortTask &t = tasks[q];
         const SortBufs &sb = *t.sb;
@@ -703,7 +759,7 @@ void launch_sort(const Geom &g, const SortTask *tasks, int ns, hipStream_t st, b
         S.clus_old = counted && t.tie && in_cell_order ? sb.clus_old : nullptr;
         S.stay = placed ? sb.stay : nullptr;
         most = t.n > most ? t.n : most;
-        big |= sb.big != nullptr;
+        if (in_cell_order && !sb.big) throw Error(-1, "a sort in cell order needs its work lists");
         if (t.n > 0 && !counted) {
             hipLaunchKernelGGL(k_hist, dim3(nblk(t.n, 256)), dim3(256), 0, st, t.keys, t.n, sb.counts);
             SMI_LAUNCH_CHECK();
@@ -728,12 +784,11 @@ void launch_sort(const Geom &g, const SortTask *tasks, int ns, hipStream_t st, b
     SMI_LAUNCH_CHECK();
     if (!in_cell_order) return;
     const int wc = fix_cells(nc * ns);
-    hipLaunchKernelGGL(k_bucket_fix, dim3(nblk(nc, 4 * wc), ns), dim3(256), 0, st, set, nc, wc, cpc, layout, G);
+    const int rank = fix_most(most, nc, nc * ns / wc);
+    hipLaunchKernelGGL(k_bucket_fix, dim3(nblk(nc, 4 * wc), ns), dim3(256), 0, st, set, nc, wc, rank, cpc, layout, G);
     SMI_LAUNCH_CHECK();
-    if (big) {
-        hipLaunchKernelGGL(k_bucket_fix_big, dim3(big_blocks(most, nc), ns), dim3(kBigThreads), 0, st, set, cpc, layout, G);
-        SMI_LAUNCH_CHECK();
-    }
+    hipLaunchKernelGGL(k_bucket_fix_big, dim3(big_blocks(most), ns), dim3(kBigThreads), 0, st, set, cpc, layout, G);
+    SMI_LAUNCH_CHECK();
 }
 
 void launch_sort(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, hipStream_t st, bool counted,
