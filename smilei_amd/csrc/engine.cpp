@@ -39,6 +39,7 @@ struct SpeciesState {
     uint32_t *keys[2] = {};        // cell keys of the particles of buffer b
     SortBufs sb{};
     int lay = 0;                   // cluster layout of sb.perm (layout_slot: 0 cell-major, 1 lane-, 2 pair-interleaved)
+    int occupied = 0;              // clusters that held particles when the species was loaded
     double *scratch = nullptr;     // 7*cap, deterministic mode
     SpeciesK k{};
     SpeciesKM km{};
@@ -93,6 +94,7 @@ struct smi_context {
     double *partials = nullptr;    // reduction scratch: kReduceBlocks for the fields and for each species
     double *rho = nullptr;         // diagnostics scratch (ncells)
     int *err = nullptr;            // device flag raised by kernels on corrupt particles
+    int *occupied = nullptr;       // device counter of sort_loaded
     int cur = 0;                   // particle buffer holding the current state
     int64_t steps = 0;             // time steps done (time_dual of the next step = (steps + 1.5) dt)
     std::vector<int> moving;       // species pushed by the next step, in id order (launch descriptors)
@@ -102,7 +104,7 @@ struct smi_context {
     int persistent = 0;            // persistent work-list form of the particle kernel (tuning)
     int cell_order = 1;            // canonical order inside a cell (atomic deposit may drop it)
     int xcd = 0;                   // XCD-aware cluster order of the grid launch (tuning)
-    int tile = 1;                  // J-tile shape of the mixed kernel: rows padded by one word (tuning)
+    int tile = 1;                  // J-tile shape of the mixed kernel: rows and planes padded (tuning)
     int tile_x = 1;                // patch-tile extent of the mixed kernel: clusters along x per workgroup (tuning)
     int node_acc = 0;              // mixed kernel: stayers' tile words summed node by node (tuning)
     bool interleave_set = false, threads_set = false, tile_set = false;  // chosen by the caller or the autotuner
@@ -132,23 +134,38 @@ void check_ctx(const smi_context *c)
     if (!c) throw Error(SMI_ERR_INVALID, "null context");
 }
 
+// Clusters with particles, of the most widespread species as loaded (of the
+// grid, before any is).
+int64_t occupied_clusters(const smi_context *c)
+{
+    int64_t most = 0;
+    for (const SpeciesState &S : c->sp) most = std::max<int64_t>(most, S.occupied);
+    return most ? most : (int64_t)c->g.npatches * c->g.clpp;
+}
+
 // Launch shape of a grid launch where nobody has chosen one (the persistent,
-// node-accumulated and two-cluster forms keep the knobs' values).  One step's particle kernel, microseconds:
-//  * Order-4 mixed form: pair-interleaved layout and unpadded J rows, whose
-//    pre-reduction halves the tile atomics that bound it: 4.2e6 particles 779
-//    against 929 lane-interleaved and padded (920 unpadded; pairs, padded 956).
+// node-accumulated and two-cluster forms keep the knobs' values).  One step's
+// particle kernel, microseconds:
+//  * Order-4 mixed form, from 768 occupied clusters (three per CU, which is what
+//    its LDS allows) on: pair-interleaved layout and unpadded J rows, whose
+//    pre-reduction halves the tile atomics that bound it.  Pairs against lanes
+//    and padded rows, 2 x 8 particles per cell: 4,096 clusters 852 / 1,001, 2,048
+//    470 / 547, 1,024 286 / 329, 512 192 / 209, but 128 122 / 103; 2 x 32: 3,365 /
+//    3,623, 1,819 / 1,924, 1,080 / 1,065, 738 / 712, 405 / 338.
 //  * Up to one cluster per CU (256) the chip is not full and 512 threads
 //    shorten each cluster's work: 16^3 cells of 2 x 8 particles, mixed order 2
 //    32 against 39 at 256 threads, FP64 48 against 58, mixed order 4 83 against
 //    98; the mixed order-2 kernel, whose workgroups are the smallest, gains up
 //    to two per CU (32^3 cells 45 against 50; FP64 90 against 80, order 4 158
 //    against 146; at three per CU 68 against 61).
-//  * 2D clusters hold 16 cells: 128 threads, unless they are crowded (256^2
-//    cells of 2 x 4 particles 58 against 84 at 256 threads, 2 x 16 116 against
-//    125, 2 x 64 405 against 384; 1024^2 cells of 2 x 16 1,575 against 1,916).
+//  * 2D clusters hold 16 cells: 128 threads, unless they are crowded.  128 / 256 /
+//    512 threads, 4,096 occupied clusters, 2 x 16 particles per cell 111 / 116 / 140,
+//    2 x 64 459 / 384 / 389, 2 x 128 1,170 / 853 / 808, 2 x 300 3,487 / 2,741 / 2,338;
+//    256 occupied of 4,096, 2 x 300 331 / 258 / 227.
 bool pair_default(const smi_context *c)
 {
-    return c->mixed && c->g.order == 4 && !c->persistent && !c->interleave_set && !c->tile_set;
+    return c->mixed && c->g.order == 4 && !c->persistent && !c->interleave_set && !c->tile_set &&
+           occupied_clusters(c) >= 768;
 }
 
 int launch_threads(const smi_context *c)
@@ -161,7 +178,8 @@ int launch_threads(const smi_context *c)
     if (g.nd == 2) {
         int64_t n = 0;
         for (int id : c->moving) n += c->sp[id].n;
-        return n <= 1024 * clusters ? 128 : 256;
+        const int64_t occupied = occupied_clusters(c);
+        return n <= 1024 * occupied ? 128 : (n <= 3072 * occupied ? 256 : 512);
     }
     return c->threads;
 }
@@ -190,14 +208,6 @@ bool want_rank(const smi_context *c)
 bool want_placed(const smi_context *c)
 {
     return c->p.deposit != SMI_DEPOSIT_DETERMINISTIC && !c->cell_order;
-}
-
-// Sort of freshly loaded particles of species S (ties: the slots themselves).
-void sort_loaded(smi_context *c, SpeciesState &S)
-{
-    S.mirrored = false;  // one buffer holds them
-    S.lay = want_interleaved(c);
-    launch_sort(c->g, S.keys[c->cur], S.n, S.sb, c->st, false, true, S.lay, nullptr, false);
 }
 
 void drop_graphs(smi_context *c)
@@ -343,6 +353,26 @@ void apply_layout(smi_context *c)
     upload_fp(c);
     upload_mix(c);
     SMI_HIP(hipStreamSynchronize(c->st));
+}
+
+// Sort of freshly loaded particles of species S (ties: the slots themselves),
+// and of how many clusters they lie in, by which the launch shape goes.
+void sort_loaded(smi_context *c, SpeciesState &S)
+{
+    S.mirrored = false;  // one buffer holds them
+    S.lay = want_interleaved(c);
+    launch_sort(c->g, S.keys[c->cur], S.n, S.sb, c->st, false, true, S.lay, nullptr, false);
+    S.occupied = 0;
+    if (S.n) {
+        launch_occupied(c->g, S.sb.cell_off, c->occupied, c->st);
+        SMI_HIP(hipMemcpyAsync(&S.occupied, c->occupied, sizeof(int), hipMemcpyDeviceToHost, c->st));
+        SMI_HIP(hipStreamSynchronize(c->st));
+    }
+    for (const SpeciesState &T : c->sp)
+        if (T.lay != want_interleaved(c)) {
+            apply_layout(c);
+            break;
+        }
 }
 
 // One PIC time step reading particle buffer c->cur and writing 1 - c->cur.
@@ -544,6 +574,7 @@ int smi_create(const smi_params *p, smi_context **out)
         c->back.init(ncells * sizeof(double));
         c->rho = dalloc<double>(ncells);
         c->err = dalloc<int>(1);
+        c->occupied = dalloc<int>(1);
         launch_fill_i32(c->err, 1, 0, c->st);
         if (p->deposit == SMI_DEPOSIT_DETERMINISTIC) c->pj = dalloc<double>(patch_j_size(g) * g.npatches);
         for (auto &e : c->ev) SMI_HIP(hipEventCreate(&e));
@@ -587,6 +618,7 @@ int smi_destroy(smi_context *c)
     (void)hipFree(c->partials);
     (void)hipFree(c->rho);
     (void)hipFree(c->err);
+    (void)hipFree(c->occupied);
     for (auto &e : c->ev)
         if (e) (void)hipEventDestroy(e);
     c->back.release();

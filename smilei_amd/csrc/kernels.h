@@ -213,6 +213,8 @@ struct SortTask {
 };
 void launch_sort(const Geom &g, const SortTask *tasks, int ns, hipStream_t st, bool counted, bool in_cell_order,
                  int layout, bool placed);
+// Number of clusters that hold particles, into *out (device).
+void launch_occupied(const Geom &g, const int32_t *cell_off, int *out, hipStream_t st);
 // Re-stores the current sorted order in another cluster layout (perm via
 // tmp); keys are those the order was sorted from.
 void launch_relayout(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, int from_layout,

@@ -691,6 +691,13 @@ __global__ void __launch_bounds__(kBigThreads) k_bucket_fix_big(SortSet set, int
     }
 }
 
+__global__ void k_occupied(const int32_t *__restrict__ cell_off, int ncl, int cpc, int *__restrict__ out)
+{
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint64_t m = __ballot(b < ncl && cell_off[(int64_t)b * cpc] != cell_off[(int64_t)(b + 1) * cpc]);
+    if ((threadIdx.x & 63) == 0 && m) atomicAdd(out, __popcll(m));
+}
+
 // Slot j of the current order, stored with cluster layout `from`, moved to
 // its slot under layout `to` (layout_slot); the cluster of the particle
 // comes from its key, cpc = cells per cluster.
@@ -796,6 +803,14 @@ void launch_sort(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, h
 {
     const SortTask one{keys, n, &sb, tie};
     launch_sort(g, &one, 1, st, counted, in_cell_order, layout, placed);
+}
+
+void launch_occupied(const Geom &g, const int32_t *cell_off, int *out, hipStream_t st)
+{
+    const int ncl = (int)(g.ncells / g.cells_per_cl);
+    launch_fill_i32(out, 1, 0, st);
+    hipLaunchKernelGGL(k_occupied, dim3(nblk(ncl, 256)), dim3(256), 0, st, cell_off, ncl, g.cells_per_cl, out);
+    SMI_LAUNCH_CHECK();
 }
 
 void launch_relayout(const Geom &g, const uint32_t *keys, int64_t n, SortBufs &sb, int from_layout,
