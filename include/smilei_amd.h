@@ -196,10 +196,12 @@ int smi_profile_step(smi_context *ctx, float *ms);
 void *smi_stream(smi_context *ctx);
 /* Launch-shape knobs of the particle kernels, searched by smi_autotune (no
  * effect on results beyond the order of the atomic J summation).  Until
- * SMI_TUNE_THREADS, or SMI_TUNE_INTERLEAVE and SMI_TUNE_TILE, are set (or the
- * autotuner has run), grid launches take the workgroup size, layout and tile
- * from the geometry and the order; the starting values that smi_get_tuning
- * reports then are those of the other launches.
+ * SMI_TUNE_THREADS, or SMI_TUNE_INTERLEAVE or SMI_TUNE_TILE, is set (or the
+ * autotuner has run), grid launches take the workgroup size, or the layout and
+ * the tile, from the geometry, the order and the loaded particles.
+ * smi_get_tuning reports the values in effect, and setting a knob to the value
+ * it reports changes nothing; setting SMI_TUNE_INTERLEAVE or SMI_TUNE_TILE to
+ * another one leaves the other of the two at its starting value (1).
  * SMI_TUNE_INTERLEAVE (mixed form and atomic FP64 form): 1 = the sort
  * stores each cluster's particles lane-interleaved (64 columns of
  * consecutive cell-sorted ranks, stored row by row), so that the 64 lanes of

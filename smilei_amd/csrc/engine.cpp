@@ -1292,6 +1292,8 @@ int smi_set_tuning(smi_context *c, int key, int value)
         if (value < 0 || value > 2) throw Error(SMI_ERR_INVALID, "SMI_TUNE_INTERLEAVE must be 0, 1 or 2");
         if (value == 2 && !c->mixed)
             throw Error(SMI_ERR_INVALID, "SMI_TUNE_INTERLEAVE = 2 (pair-interleaved) is a mixed-form layout");
+        // (the layout in effect: its tile stays too)
+        if (value == want_interleaved(c)) c->tile = launch_tile(c);
         c->interleave = value;
         c->interleave_set = true;
     } else if (key == SMI_TUNE_THREADS) {
@@ -1310,6 +1312,8 @@ int smi_set_tuning(smi_context *c, int key, int value)
         c->persistent = value != 0;
     } else if (key == SMI_TUNE_TILE) {
         if (value != 0 && value != 1) throw Error(SMI_ERR_INVALID, "SMI_TUNE_TILE must be 0 or 1");
+        // (the tile in effect: its layout stays too)
+        if (value == launch_tile(c) && pair_default(c)) c->interleave = want_interleaved(c);
         c->tile = value;
         c->tile_set = true;
     } else if (key == SMI_TUNE_TILE_X) {
@@ -1339,11 +1343,11 @@ int smi_get_tuning(smi_context *c, int key, int *value)
     SMI_TRY
     check_ctx(c);
     if (!value) throw Error(SMI_ERR_INVALID, "null output");
-    if (key == SMI_TUNE_INTERLEAVE) *value = c->interleave;
-    else if (key == SMI_TUNE_THREADS) *value = c->threads;
+    if (key == SMI_TUNE_INTERLEAVE) *value = pair_default(c) ? want_interleaved(c) : c->interleave;
+    else if (key == SMI_TUNE_THREADS) *value = launch_threads(c);
     else if (key == SMI_TUNE_PERSISTENT) *value = c->persistent;
     else if (key == SMI_TUNE_XCD) *value = c->xcd;
-    else if (key == SMI_TUNE_TILE) *value = c->tile;
+    else if (key == SMI_TUNE_TILE) *value = launch_tile(c);
     else if (key == SMI_TUNE_TILE_X) *value = c->tile_x;
     else if (key == SMI_TUNE_NODE_ACC) *value = c->node_acc;
     else if (key == SMI_TUNE_CELL_ORDER) *value = c->cell_order || c->p.deposit == SMI_DEPOSIT_DETERMINISTIC;
