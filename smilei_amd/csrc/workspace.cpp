@@ -9,15 +9,22 @@ namespace smi {
 
 namespace {
 
+// A device's pool: made at the first use, held until the process ends.
+struct DevicePool {
+    hipMemPool_t pool = nullptr;
+    bool tried = false;  // a device without pools is not asked again
+};
 
 std::mutex g_lock;
-std::vector<hipMemPool_t> g_pool;  // by device; made at the first use, held until the process ends
+std::vector<DevicePool> g_pool;  // by device
 
 hipMemPool_t device_pool(int dev)
 {
     std::lock_guard<std::mutex> hold(g_lock);
-    if ((int)g_pool.size() <= dev) g_pool.resize(dev + 1, nullptr);
-    if (!g_pool[dev]) {
+    if ((int)g_pool.size() <= dev) g_pool.resize(dev + 1);
+    DevicePool &d = g_pool[dev];
+    if (!d.tried) {
+        d.tried = true;
         hipMemPoolProps props{};
         props.allocType = hipMemAllocationTypePinned;
         props.location.type = hipMemLocationTypeDevice;
@@ -25,29 +32,37 @@ hipMemPool_t device_pool(int dev)
         hipMemPool_t pool = nullptr;
         if (hipMemPoolCreate(&pool, &props) != hipSuccess) return nullptr;
         uint64_t keep = kWorkspaceKeep;
-        (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-        g_pool[dev] = pool;
+        // (without its threshold a pool only gives everything back)
+        if (hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep) != hipSuccess) (void)hipGetLastError();
+        d.pool = pool;
     }
-    return g_pool[dev];
+    return d.pool;
+}
+
+bool allocate(void **p, size_t bytes, hipStream_t st)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return false;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    const hipMemPool_t pool = device_pool(dev);
+    return pool && hipMallocFromPoolAsync(p, bytes, pool, st) == hipSuccess;
 }
 
 }  // namespace
 
 Workspace::Workspace(size_t bytes, hipStream_t stream) : st(stream)
 {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone) return;
-    int dev = 0;
-    hipMemPool_t pool = hipGetDevice(&dev) == hipSuccess ? device_pool(dev) : nullptr;
-    if (pool && hipMallocFromPoolAsync(&p, bytes, pool, stream) != hipSuccess) {
-        p = nullptr;
-        (void)hipGetLastError();  // out of memory: the caller does without
-    }
+    if (allocate(&p, bytes, stream)) return;
+    p = nullptr;
+    // the caller does without: what failed here must not be taken for a
+    // failure of the launches that follow
+    (void)hipGetLastError();
 }
 
 Workspace::~Workspace()
 {
-    if (p) (void)hipFreeAsync(p, st);
+    if (p && hipFreeAsync(p, st) != hipSuccess) (void)hipGetLastError();
 }
 
 }  // namespace smi
