@@ -214,8 +214,9 @@ __global__ void k_ukin(PartPtrs A, const int32_t *__restrict__ perm, int64_t n, 
 // contribution to global memory instead was bound by the memory-side FP64
 // atomics (27 or 125 per particle, 3e10/s): mean 1.71 ms over species of
 // 2.4e6, 2.4e6 and 6.2e5 particles at order 2, 1.70 ms for 4.1e5 at order 4,
-// 1.30 ms for 4.2e6 in 2D, against 0.053, 0.059 and 0.036 ms for the tile.  A node outside the tile (a position its key does
-// not describe) goes to global memory directly.
+// 1.30 ms for 4.2e6 in 2D, against 0.053, 0.059 and 0.036 ms for the tile.  A
+// node outside the tile (a position its key does not describe) goes to global
+// memory directly.
 template <int ND, int ORDER>
 __global__ void __launch_bounds__(256)
 k_rho(Geom g, SpeciesK sp, PartPtrs A, const int32_t *__restrict__ perm, const int32_t *__restrict__ cell_off,

@@ -182,9 +182,9 @@ __global__ void __launch_bounds__(128, 2) k_proj3d_atomic(Proj3Args a)
 }
 
 // The same currents over particles binned by their old node: bin = the 4^3
-// nodes it lies in.  One workgroup per bin sums its particles' stencils (a
-// tile of 6 + 2H points per axis) in LDS and flushes the tile once, instead
-// of adding 54 to 400 contributions per particle to global memory, which the
+// nodes it lies in.  One workgroup per bin, or per share of a crowded one, sums
+// its particles' stencils (a tile of 6 + 2H points per axis) in LDS and flushes
+// the tile once, instead of adding 54 to 400 contributions per particle to global memory, which the
 // memory-side FP64 atomics bound at 4e10 per second whatever the order of
 // the particles.  The particles are not moved: the bins list their indices.
 // The strides of the tile put the 64 nodes of a bin, at one stencil offset,
@@ -886,7 +886,7 @@ __global__ void __launch_bounds__(256, 3) k_interp3d_bins(Interp3Args a, Bins b)
 // k_interp3d against bins: 2.6e5 particles 83 / 205 us against 95 / 142; 5.1e5 159
 // / 455 against 146 / 220; 1.0e6, 180 to a bin, 282 / 1,733 against 261 / 378;
 // 2.1e6 524 / 4,002 against 415 / 853; but 5.2e5, 90 to a bin, 143 against 195 in
-// cell order.  Order 2, 2.1e6: 144 / 886 against 166 / 466, left as it is.
+// cell order.  6e5 within 2^3 cells: 260 / 299 against 133 / 145.  Order 2, 2.1e6: 144 / 886 against 166 / 466, left as it is.
 constexpr int64_t kInterpBinMin = 1 << 19, kInterpPerBin = 160;
 
 bool launch_interp_bins(int order, const Interp3Args &a, hipStream_t st)

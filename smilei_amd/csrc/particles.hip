@@ -160,9 +160,10 @@ __device__ __attribute__((always_inline)) inline void fp_cluster(const Geom &g, 
     __shared__ double sF[6 * GF];
     __shared__ double sJ[DEPOSIT ? 3 * JSC : 1];
     __shared__ int sHist[kMaxMerged][64];  // destination-cell counts of this cluster's own cells
-    // particles whose node changes on some axis are deposited in a second pass over this queue (old delta, new position in cells, charge
-    // weight, old node relative to the cluster), so that the main loop runs
-    // the narrow stencil with all lanes.  Order 4: a short queue, so that the
+    // particles whose node changes on some axis are deposited in a second pass
+    // over this queue (old delta, new position in cells, charge weight, old node
+    // relative to the cluster), so that the main loop runs the narrow stencil
+    // with all lanes.  Order 4: a short queue, so that the
     // workgroup's LDS (field and J tiles of 10^3 and 11^3 points) stays within
     // 80 KB and two workgroups fit a CU.
     constexpr int QCAP = DEPOSIT ? (ORDER == 4 ? 12 : 96) : 1;

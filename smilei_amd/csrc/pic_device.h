@@ -1,7 +1,9 @@
 // pic_device.h -- device arithmetic shared by the batched kernels and the
 // per-operator entry points: Boris push, B-spline gathers and the Esirkepov
-// current contributions, each in the association order of the reference
-// operator it restates (the library is built with -ffp-contract=off).
+// current contributions.  boris, gather2/3/3s and esirkepov2d/3d keep the
+// association order of the reference operator they restate (the library is built
+// with -ffp-contract=off); boris_fused, gather2/3_fused and esirkepov3d_fact,
+// whose callers promise no order of sums, are factorised and fused.
 #pragma once
 
 #include "common.h"
@@ -473,12 +475,10 @@ __device__ inline void esirkepov3d(const double (&S0)[3][7], const double (&DS)[
 // entries of the reference's ORDER+3-entry stencil, starting at w0 = 0 when
 // sh < 0 and at w0 = 1 otherwise.  Outside the window S0 = DS = 0 exactly,
 // so the skipped columns contribute exact zeros, and the prefix sums along
-// the current's axis start from an exact zero: the values added below are
-// bit-identical to the reference's.  The window arrays are filled with
-// compile-time indices only (selects, no dynamic register indexing).
+// the current's axis start from an exact zero.  The window arrays are filled
+// with compile-time indices only (selects, no dynamic register indexing).
 template <int ORDER>
-__device__ inline void esirkepov_window(double dold, double pn_new, int ipo, double *S0w, double *DSw, int &w0,
-                                        int *shift = nullptr)
+__device__ inline void esirkepov_window(double dold, double pn_new, int ipo, double *S0w, double *DSw, int &w0)
 {
     constexpr int W = ORDER + 2;
     double s[ORDER + 1], nw[ORDER + 1];
@@ -487,7 +487,6 @@ __device__ inline void esirkepov_window(double dold, double pn_new, int ipo, dou
     spline<ORDER>(pn_new - (double)ip, nw);
     const int sh = ip - ipo;
     w0 = sh < 0 ? 0 : 1;
-    if (shift) *shift = sh;
 #pragma unroll
     for (int m = 0; m < W; ++m) {
         const double s0_w0 = m == 0 ? 0. : s[m - 1];     // window starting at stencil 0

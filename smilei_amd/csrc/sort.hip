@@ -303,7 +303,7 @@ __global__ void __launch_bounds__(kScatThreads) k_scatter(SortSet set, int cpc, 
 }
 
 // Canonical order inside a cell: by direction of motion, then source slot.
-// A wavefront takes 64 cells, whose particles are one run of places, and works
+// A wavefront takes 16 to 64 cells, whose particles are one run of places, and works
 // on as many whole cells at a time as fit into kFixBatch places: one lane per
 // place, kFixPer places per lane in flight.  The keys are staged in LDS, and a
 // lane's rank is the number of smaller (direction, slot) pairs of its cell; the
