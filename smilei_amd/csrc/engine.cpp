@@ -91,7 +91,8 @@ struct smi_context {
     int d_det_n = 0;
     MixSpecies *d_mix = nullptr;   // mixed-form particle-launch descriptors [2][species]
     FpSpecies *d_fp = nullptr;     // FP64-form particle-launch descriptors [2][species]
-    double *partials = nullptr;    // reduction scratch: kReduceBlocks for the fields and for each species
+    double *partials = nullptr;    // reduction scratch: kReduceBlocks for the fields and for each species ...
+    int64_t partials_for = 0;      // ... up to this many
     double *rho = nullptr;         // diagnostics scratch (ncells)
     int *err = nullptr;            // device flag raised by kernels on corrupt particles
     int *occupied = nullptr;       // device counter of sort_loaded
@@ -570,7 +571,8 @@ int smi_create(const smi_params *p, smi_context **out)
             c->F[f] = dalloc<double>(ncells);
             launch_fill(c->F[f], ncells, 0.0, c->st);
         }
-        c->partials = dalloc<double>(kReduceBlocks);
+        c->partials_for = 4;
+        c->partials = dalloc<double>((1 + c->partials_for) * kReduceBlocks);
         c->back.init(ncells * sizeof(double));
         c->rho = dalloc<double>(ncells);
         c->err = dalloc<int>(1);
@@ -672,10 +674,13 @@ int smi_add_species(smi_context *c, const char *name, double mass, double charge
     s.km.cwd = s.k.cw_scale;
     for (int d = 0; d < 3; ++d) s.km.dxdt[d] = (float)(c->g.dx[d] / c->g.dt);
     set_quantum(c->g, s, 1.0);
-    double *partials = dalloc<double>((2 + (int64_t)c->sp.size()) * kReduceBlocks);
-    SMI_HIP(hipStreamSynchronize(c->st));
-    (void)hipFree(c->partials);
-    c->partials = partials;
+    if ((int64_t)c->sp.size() == c->partials_for) {
+        double *partials = dalloc<double>((1 + 2 * c->partials_for) * kReduceBlocks);
+        SMI_HIP(hipStreamSynchronize(c->st));
+        (void)hipFree(c->partials);
+        c->partials = partials;
+        c->partials_for *= 2;
+    }
     c->sp.push_back(s);
     c->moving = moving_now(c);
     // deterministic-deposit descriptors for both ping-pong parities
