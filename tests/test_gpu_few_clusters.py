@@ -47,7 +47,9 @@ def test_untouched_knobs_cost_no_more(case):
     else:
         args, by_hand = ((64, 64, 64), (12, 12, 12), 300), [(sa.TUNE_INTERLEAVE, 1), (sa.TUNE_TILE, 1)]
         kw = dict(order=4, form=sa.MIXED)
-    assert kernel_ms(plasma(*args, **kw)) <= 1.1 * kernel_ms(plasma(*args, tuning=by_hand, **kw))
+    times = [[kernel_ms(plasma(*args, tuning=t, **kw)) for t in ((), by_hand)] for _ in range(3)]
+    untouched, hand = (min(t) for t in zip(*times))
+    assert untouched <= 1.1 * hand
 
 
 @pytest.mark.parametrize("widespread", [False, True])

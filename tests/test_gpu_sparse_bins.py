@@ -31,7 +31,9 @@ def per_call(n):
 
 @pytest.mark.parametrize("n", [(75, 75, 75), (77, 77, 77)])
 def test_few_particles_to_a_bin_cost_no_more(n):
-    assert per_call(n) <= 1.07 * per_call((83, 83, 83))
+    times = [[per_call(k) for k in (n, (83, 83, 83))] for _ in range(2)]
+    here, more_bins = (min(t) for t in zip(*times))
+    assert here <= 1.07 * more_bins
 
 
 @pytest.mark.parametrize("n,m", [((75, 75, 75), 11999), ((75, 75, 75), 12000), ((60, 76, 72), 9000)])
